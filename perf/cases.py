@@ -51,8 +51,8 @@ def listed():
         # with the engine's default sort interval
         dict(name="frame_snow_500k", kind="frame", scene="snow", particles=500_000, N=64, substeps=42,
              sort_every=16),
-        # a dense elastic body, every second frame saved
-        dict(name="run_elastic_200k", kind="frame", scene="elastic", particles=200_000, N=64, substeps=84,
+        # a dense elastic body at a longer sort interval
+        dict(name="frame_elastic_200k", kind="frame", scene="elastic", particles=200_000, N=64, substeps=42,
              sort_every=32),
         # the dam break, the benchmark's headline scene: a frame of 83 substeps
         dict(name="frame_liquid_1m", kind="frame", scene="liquid", particles=1_000_000, N=128, substeps=83,
@@ -85,7 +85,7 @@ def draw(rng):
         n = log_int(3_000, 1_000_000)
         # 2 to 60 particles a cell of the body, which fills about a tenth of the box
         N = int(min(128, max(16, round((n / (0.1 * rng.uniform(2.0, 60.0))) ** (1 / 3)))))
-        k = log_int(8, {"liquid": 400, "elastic": 84}.get(scene, 48))
+        k = log_int(8, 400 if scene == "liquid" else 48)
         return dict(kind="frame", scene=scene, particles=n, N=N, substeps=k, sort_every=rng.choice([16, 32, 48, 96]))
     if kind == "batch":
         return dict(kind="batch", scenes=rng.randint(3, 24), max_particles=log_int(8_000, 120_000),
