@@ -179,8 +179,17 @@ class Sim {
   int upload_materials();
   int sort_particles(hipStream_t s);
   int substep(hipStream_t s);
-  int fetch_state(std::vector<float>& planes, std::vector<uint8_t>& mat,
-                  std::vector<uint32_t>& id, hipStream_t s);
+  // device bytes [0, bytes) to the host: `take` gets every chunk once it is in
+  // pinned memory (offset, data, size), from several threads for large ones
+  template <class Take>
+  int fetch_chunks(const uint8_t* src, size_t bytes, const Take& take, hipStream_t s);
+  // pinned slots of fetch_chunks, each with the event of its last copy; at
+  // most kStageSlots of kStageBytes a handle
+  static constexpr int kStageSlots = 8;
+  static constexpr size_t kStageBytes = (size_t)4 << 20;
+  uint8_t* h_stage_[kStageSlots] = {};
+  size_t stage_bytes_[kStageSlots] = {};
+  hipEvent_t stage_ev_[kStageSlots] = {};
   int hip_fail(hipError_t e, const char* what);
   int check_materials_cover_particles(const char* who);
   // timing: events recorded around a phase when opt_.timing is set

@@ -69,6 +69,11 @@ hipError_t build_items(const uint32_t* keys, const uint32_t* perm, int64_t n, in
 hipError_t remove_range(const ParticlesDev& src, const ParticlesDev& dst, uint32_t lo, uint32_t hi,
                         uint32_t* flag, uint32_t* pos, uint32_t* scratch, uint32_t* total, float* gone,
                         uint8_t* gone_mat, hipStream_t s);
+// The particle state in original-index order: rows of x, v, C, F, Jp (25 n
+// floats, array after array) and the n materials. *bad is set when an index
+// is not below n. derive: F = cbrt(Jp) I instead of the F planes.
+hipError_t export_state(const ParticlesDev& P, float* out, uint8_t* mat, uint32_t* bad, int derive,
+                        hipStream_t s);
 // dst[i] = src[perm[i]]
 hipError_t reorder(const ParticlesDev& src, const ParticlesDev& dst, const uint32_t* perm,
                    hipStream_t s);

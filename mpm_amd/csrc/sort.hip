@@ -21,6 +21,8 @@
 //                    digits, per-wave counts in LDS), then scatter
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "device_math.hpp"
 #include "engine_types.hpp"
 #include "kernels.hpp"
@@ -574,6 +576,59 @@ __global__ void __launch_bounds__(256)
   dst.id[j] = id >= hi ? id - (hi - lo) : id;
 }
 
+// The state in original-index order, as downloads hand it out: rows x (3), v
+// (3), C (9), F (9), Jp of particle id at out + {0, 3n, 6n, 15n, 24n}, its
+// material at mat + id. An id past n (none is ever made) sets *bad instead.
+// derive: F = cbrt(Jp) I (the liquid's implicit F, the bits of k_liquid_f).
+// Bound by its scattered stores: the ids of neighbouring slots are far apart,
+// so a row of 36 bytes is the longest run there is. A workgroup turns its 256
+// particles' planes into rows through LDS and neighbouring lanes store
+// neighbouring words of a row, 7 rows of C per store instead of 64 lines.
+constexpr int kExportThreads = 256;
+__global__ void __launch_bounds__(kExportThreads)
+    k_export(ParticlesDev P, float* __restrict__ out, uint8_t* __restrict__ mat, uint32_t* __restrict__ bad,
+             int derive) {
+  constexpr int T = kExportThreads;
+  __shared__ float t[NUM_PLANES][T + 1];
+  __shared__ uint32_t ids[T];
+  const int64_t n = P.n;
+  const int64_t i = (int64_t)blockIdx.x * T + threadIdx.x;
+  uint32_t id = 0xffffffffu;  // past every n: nothing is stored
+  if (i < n) {
+    id = P.id[i];
+    if ((int64_t)id < n) mat[id] = P.mat[i];
+    else *bad = 1u;
+#pragma unroll
+    for (int p = 0; p < PL_F; ++p) t[p][threadIdx.x] = P.f[(size_t)p * P.stride + i];
+    const float jp = P.f[(size_t)PL_JP * P.stride + i];
+    t[PL_JP][threadIdx.x] = jp;
+    if (derive) {
+      const float cj = cbrtf(jp);
+#pragma unroll
+      for (int a = 0; a < 9; ++a) t[PL_F + a][threadIdx.x] = (a % 4 == 0) ? cj : 0.0f;
+    } else {
+#pragma unroll
+      for (int a = 0; a < 9; ++a) t[PL_F + a][threadIdx.x] = P.f[(size_t)(PL_F + a) * P.stride + i];
+    }
+  }
+  ids[threadIdx.x] = id;
+  __syncthreads();
+  const auto rows = [&](int plane, auto width) {
+    constexpr int W = decltype(width)::value;
+    float* const dst = out + (size_t)plane * n;
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+      const int e = j * T + (int)threadIdx.x, p = e / W, c = e - p * W;
+      if ((int64_t)ids[p] < n) dst[(size_t)ids[p] * W + c] = t[plane + c][p];
+    }
+  };
+  rows(PL_X, std::integral_constant<int, 3>{});
+  rows(PL_V, std::integral_constant<int, 3>{});
+  rows(PL_C, std::integral_constant<int, 9>{});
+  rows(PL_F, std::integral_constant<int, 9>{});
+  rows(PL_JP, std::integral_constant<int, 1>{});
+}
+
 template <int BITS>
 hipError_t radix_sort_t(uint32_t* keys[2], uint32_t* vals[2], int64_t n, int start_bit, int key_bits,
                         uint32_t* scratch, int* out_idx, hipStream_t s) {
@@ -776,6 +831,15 @@ hipError_t remove_range(const ParticlesDev& src, const ParticlesDev& dst, uint32
   hipError_t e = exclusive_scan(flag, pos, src.n, scratch, total, s);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_compact, dim3(g), dim3(256), 0, s, src, dst, pos, lo, hi, gone, gone_mat);
+  return hipGetLastError();
+}
+
+hipError_t export_state(const ParticlesDev& P, float* out, uint8_t* mat, uint32_t* bad, int derive,
+                        hipStream_t s) {
+  if (P.n <= 0) return hipSuccess;
+  if (!out || !mat || !bad) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_export, dim3((unsigned)((P.n + kExportThreads - 1) / kExportThreads)),
+                     dim3(kExportThreads), 0, s, P, out, mat, bad, derive);
   return hipGetLastError();
 }
 
