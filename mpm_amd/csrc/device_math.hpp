@@ -514,6 +514,17 @@ __device__ __forceinline__ void polar_rotation(const float* F, float* R) {
   mul_abt(U, V, R);
 }
 
+// Inclusive max-scan over the lanes of a wavefront with DPP (no LDS traffic).
+__device__ __forceinline__ int wave_max_scan(int v) {  // v >= 0
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111 /* row_shr:1 */, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112 /* row_shr:2 */, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114 /* row_shr:4 */, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118 /* row_shr:8 */, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142 /* row_bcast:15 */, 0xa, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143 /* row_bcast:31 */, 0xc, 0xf, true));
+  return v;
+}
+
 // ---------------------------------------------------------------------------
 // Multi-scene launches: index g (a workgroup or a block of the launch) lies in
 // scene j when prefix[j] <= g < prefix[j + 1]. Every lane of the wavefront

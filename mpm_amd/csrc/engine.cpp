@@ -636,7 +636,8 @@ int Sim::mesh_build(int side, int radius, int64_t* ntri, hipStream_t s) {
   const double vdx = (double)((float)k_.N * k_.dx) / (double)side;
   const float vdx_f = (float)vdx, cutoff = (float)((double)(radius + 1) * vdx);
   const double rv = (double)radius * vdx;
-  const size_t nv = (size_t)side * side * side, nc = (size_t)(side - 1) * (side - 1) * (side - 1);
+  const size_t nv = (size_t)side * side * side, ncubes = (size_t)(side - 1) * (side - 1) * (side - 1);
+  const size_t nb = (size_t)mpmk::mesh_bins(side), nc = std::max(ncubes, nb * nb * nb);
   if (nv > sdf_cap_) {
     if (d_sdf_) (void)hipFree(d_sdf_);
     d_sdf_ = nullptr;
@@ -656,10 +657,16 @@ int Sim::mesh_build(int side, int radius, int64_t* ntri, hipStream_t s) {
     HIPCHK(hipMalloc(&d_mscratch_, sizeof(uint32_t) * (nc / 2048 + 2)), "hipMalloc(mesh scan)");
     mcube_cap_ = nc;
   }
-  HIPCHK(mpmk::mesh_distance_field(particles(), side, vdx_f, cutoff, d_sdf_, s), "mesh distance field");
+  // the bins use the cubes' arrays before the cubes do, and the particle copy
+  // that the next reorder overwrites
+  float* const other = d_f_[cur_ ^ 1];
+  const mpmk::MeshScratch w{d_mcount_, d_moff_, d_mscratch_, other ? (uint32_t*)(other + 3 * stride_) : nullptr,
+                            other, stride_};
+  const double fill = std::min(1.0, (double)std::max<int64_t>(1, occupied_) / (double)node_blocks());
+  HIPCHK(mpmk::mesh_distance_field(particles(), side, vdx_f, cutoff, fill, w, d_sdf_, s), "mesh distance field");
   HIPCHK(mpmk::mesh_count(d_sdf_, side, rv, d_mcount_, s), "mesh count");
-  uint32_t* total = d_moff_ + nc;
-  HIPCHK(mpmk::exclusive_scan(d_mcount_, d_moff_, (int64_t)nc, d_mscratch_, total, s), "mesh scan");
+  uint32_t* total = d_moff_ + ncubes;
+  HIPCHK(mpmk::exclusive_scan(d_mcount_, d_moff_, (int64_t)ncubes, d_mscratch_, total, s), "mesh scan");
   uint32_t n = 0;
   HIPCHK(hipMemcpyAsync(&n, total, sizeof(uint32_t), hipMemcpyDeviceToHost, s), "mesh size");
   HIPCHK(hipStreamSynchronize(s), "mesh size");

@@ -225,8 +225,21 @@ hipError_t tile_combine(const TileSums& in, int64_t nblk, hipStream_t s);
 // triangle count of each of the (side-1)^3 cubes of S = rv - distance = 0,
 // mesh_emit writes them (9 floats each, and the 3 grid edges their
 // vertices lie on) at the scanned offsets.
-hipError_t mesh_distance_field(const ParticlesDev& P, int side, float vdx, float cutoff, uint32_t* sdf,
-                               hipStream_t s);
+// Scratch of the field: mesh_bins(side)^3 counts, one start more, the scan's
+// tile sums (one per 2048 counts), a rank and 3 planes of pos_stride floats
+// for the particles.
+struct MeshScratch {
+  uint32_t* count;
+  uint32_t* start;
+  uint32_t* scan;
+  uint32_t* rank;
+  float* pos;
+  size_t pos_stride;
+};
+int mesh_bins(int side);
+// `fill`: share of the box that holds particles, as far as is known
+hipError_t mesh_distance_field(const ParticlesDev& P, int side, float vdx, float cutoff, double fill,
+                               const MeshScratch& w, uint32_t* sdf, hipStream_t s);
 hipError_t mesh_count(const uint32_t* sdf, int side, double rv, uint32_t* count, hipStream_t s);
 hipError_t mesh_emit(const uint32_t* sdf, int side, double rv, double vdx, const uint32_t* offset, float* xyz,
                      uint64_t* keys, hipStream_t s);

@@ -222,23 +222,13 @@ __device__ __forceinline__ void scatter_global(const float q0[3][3], const float
 // Material-kind sets compiled into an instantiation.
 enum KindSet : int { KINDS_ALL = 0, KINDS_LIQUID = 1 };
 
-// Wavefront lane shifts and an inclusive max-scan with DPP (no LDS traffic).
+// Wavefront lane shifts with DPP (no LDS traffic).
 __device__ __forceinline__ int dpp_wave_shr1(int v) {  // lane l gets lane l-1; lane 0 gets 0
   return __builtin_amdgcn_update_dpp(0, v, 0x138 /* wave_shr:1 */, 0xf, 0xf, true);
 }
 __device__ __forceinline__ int dpp_wave_shl1(int v) {  // lane l gets lane l+1; lane 63 gets 0
   return __builtin_amdgcn_update_dpp(0, v, 0x130 /* wave_shl:1 */, 0xf, 0xf, true);
 }
-__device__ __forceinline__ int wave_max_scan(int v) {  // v >= 0
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111 /* row_shr:1 */, 0xf, 0xf, true));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112 /* row_shr:2 */, 0xf, 0xf, true));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114 /* row_shr:4 */, 0xf, 0xf, true));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118 /* row_shr:8 */, 0xf, 0xf, true));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142 /* row_bcast:15 */, 0xa, 0xf, true));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143 /* row_bcast:31 */, 0xc, 0xf, true));
-  return v;
-}
-
 // LDS slot of tile node (x, y, z) in an 8^3 tile: z is permuted within its
 // row (bit 2 flipped when x + y is odd), so the runs of 4 neighbouring nodes
 // that the lanes of one access touch in adjacent rows or planes land in

@@ -70,6 +70,35 @@ def test_distance_field_matches_oracle(gpu_lib):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("n,side,r,N", [
+    # gathered
+    (200, 2, 2, 32),      # one partial block of voxels
+    (2000, 5, 2, 32),     # ragged blocks
+    (3000, 31, 2, 24),    # one shell of blocks
+    (1500, 50, 5, 24),    # the mesher's default radius, two shells
+    (700, 37, 9, 32),     # three shells
+    (60_000, 22, 4, 32),  # hundreds in a bin: 4 wavefronts a block
+    (90_000, 16, 3, 32),  # thousands: 16
+    # scattered
+    (600, 40, 17, 32),    # a box edge of 37 voxels
+    (40, 120, 0, 32),     # small boxes
+    (9000, 12, 1, 32),    # crowded bins
+])
+def test_distance_field_over_its_paths(gpu_lib, n, side, r, N):
+    rng = np.random.default_rng(n)
+    x = rng.uniform(-0.08, 1.08, (n, 3))
+    # a crowded corner, and particles on voxel nodes: distances equal to the
+    # cut-off, where the truncated box decides
+    x[: n // 4] = 0.3 + 0.1 * rng.random((n // 4, 3))
+    x[n // 2:] = np.where(rng.random((n - n // 2, 1)) < 0.3, np.round(x[n // 2:] * side) / side, x[n // 2:])
+    x = x.astype(np.float32)
+    e = engine_with(x, N)
+    e.mesh(side, r)
+    got = e.mesh_distance_field(side)
+    e.close()
+    assert np.array_equal(got, distance_field(x, N, side, r))
+
+
 def test_marching_cubes_matches_oracle(gpu_lib):
     from oracle.mesh import marching_cubes
     N, side, r = 32, 40, 3
