@@ -624,6 +624,103 @@ int Sim::remove(int64_t first, int64_t count, void* removed, hipStream_t s) {
   return MPM_OK;
 }
 
+// The bytes pass through pinned slots, whose copies run at the link's rate
+// (about 50 GB/s here; straight into pageable memory they run at 10). Taking
+// a chunk out of its slot is the slow part: the caller's arrays are mostly
+// new memory, whose pages the system hands out one fault at a time, at 3 to 5
+// GB/s a thread. So one thread for every 2 MB, up to one a slot, takes
+// chunks, while this one keeps the copies queued on s.
+template <class Take>
+int Sim::fetch_chunks(const uint8_t* src, size_t bytes, const Take& take, hipStream_t s) {
+  if (bytes == 0) return MPM_OK;
+  const size_t cores = std::max(1u, std::thread::hardware_concurrency());
+  size_t slots = std::min({(size_t)kStageSlots, cores, (bytes + ((size_t)2 << 20) - 1) >> 21});
+  const size_t chunk = std::min(kStageBytes, ((bytes + slots - 1) / slots + 4095) & ~(size_t)4095);
+  for (size_t w = 0; w < slots; ++w) {
+    if (stage_bytes_[w] < chunk) {
+      if (h_stage_[w]) (void)hipHostFree(h_stage_[w]);
+      h_stage_[w] = nullptr;
+      stage_bytes_[w] = 0;
+      HIPCHK(hipHostMalloc((void**)&h_stage_[w], chunk, 0), "hipHostMalloc(download)");
+      stage_bytes_[w] = chunk;
+    }
+    if (!stage_ev_[w]) HIPCHK(hipEventCreateWithFlags(&stage_ev_[w], hipEventDisableTiming), "hipEventCreate");
+  }
+  const size_t n = (bytes + chunk - 1) / chunk;
+  const auto size_of = [&](size_t c) { return std::min(chunk, bytes - c * chunk); };
+  const auto queue = [&](size_t c) {
+    const size_t w = c % slots;
+    hipError_t e = hipMemcpyAsync(h_stage_[w], src + c * chunk, size_of(c), hipMemcpyDeviceToHost, s);
+    return e == hipSuccess ? hipEventRecord(stage_ev_[w], s) : e;
+  };
+  std::mutex m;
+  std::condition_variable cv;
+  size_t queued = 0;                       // chunks whose copies are on the stream (under m, as the rest)
+  bool stop = false;
+  std::vector<size_t> taken(slots, 0);     // chunks taken out of each slot
+  std::vector<hipError_t> bad(slots, hipSuccess);
+  // slot w's thread: chunks w, w + slots, ...
+  const auto work = [&](size_t w) {
+    hipError_t e = hipSetDevice(device_);
+    for (size_t c = w; c < n; c += slots) {
+      {
+        std::unique_lock<std::mutex> lock(m);
+        cv.wait(lock, [&] { return queued > c || stop; });
+        if (queued <= c) return;
+      }
+      if (e == hipSuccess) e = hipEventSynchronize(stage_ev_[w]);
+      if (e == hipSuccess) take(c * chunk, h_stage_[w], size_of(c));
+      std::lock_guard<std::mutex> lock(m);
+      ++taken[w];
+      bad[w] = e;
+      cv.notify_all();
+    }
+  };
+  std::vector<std::thread> threads;
+  if (slots > 1) {
+    try {
+      for (size_t w = 0; w < slots; ++w) threads.emplace_back(work, w);
+    } catch (const std::exception&) {
+      // no more threads to be had: those that started end, and one slot does
+      {
+        std::lock_guard<std::mutex> lock(m);
+        stop = true;
+      }
+      cv.notify_all();
+      for (auto& t : threads) t.join();
+      threads.clear();
+      slots = 1;
+    }
+  }
+  hipError_t e = hipSuccess;
+  if (threads.empty()) {
+    for (size_t c = 0; c < n && e == hipSuccess; ++c) {
+      e = queue(c);
+      if (e == hipSuccess) e = hipEventSynchronize(stage_ev_[c % slots]);
+      if (e == hipSuccess) take(c * chunk, h_stage_[c % slots], size_of(c));
+    }
+    HIPCHK(e, "download");
+    return MPM_OK;
+  }
+  for (size_t c = 0; c < n && e == hipSuccess; ++c) {
+    const size_t w = c % slots;
+    {
+      std::unique_lock<std::mutex> lock(m);
+      cv.wait(lock, [&] { return taken[w] == c / slots || bad[w] != hipSuccess; });
+      e = bad[w];
+    }
+    if (e == hipSuccess) e = queue(c);
+    std::lock_guard<std::mutex> lock(m);
+    if (e == hipSuccess) queued = c + 1;
+    else stop = true;
+    cv.notify_all();
+  }
+  for (auto& t : threads) t.join();
+  for (size_t w = 0; w < slots && e == hipSuccess; ++w) e = bad[w];
+  HIPCHK(e, "download");
+  return MPM_OK;
+}
+
 // Surface mesh (mesh.hip) of the device particles, as the reference's
 // MeshBuilder::computeMesh does it on the host (mesh_builder.h:181-211):
 // voxel_dx = N dx / side (float N dx, then double), distance cut-off
@@ -636,8 +733,8 @@ int Sim::mesh_build(int side, int radius, int64_t* ntri, hipStream_t s) {
   const double vdx = (double)((float)k_.N * k_.dx) / (double)side;
   const float vdx_f = (float)vdx, cutoff = (float)((double)(radius + 1) * vdx);
   const double rv = (double)radius * vdx;
-  const size_t nv = (size_t)side * side * side, ncubes = (size_t)(side - 1) * (side - 1) * (side - 1);
-  const size_t nb = (size_t)mpmk::mesh_bins(side), nc = std::max(ncubes, nb * nb * nb);
+  const size_t nv = (size_t)side * side * side, rows = (size_t)(side - 1) * (side - 1);
+  const size_t nb = (size_t)mpmk::mesh_bins(side), nc = std::max(rows, nb * nb * nb);
   if (nv > sdf_cap_) {
     if (d_sdf_) (void)hipFree(d_sdf_);
     d_sdf_ = nullptr;
@@ -657,7 +754,7 @@ int Sim::mesh_build(int side, int radius, int64_t* ntri, hipStream_t s) {
     HIPCHK(hipMalloc(&d_mscratch_, sizeof(uint32_t) * (nc / 2048 + 2)), "hipMalloc(mesh scan)");
     mcube_cap_ = nc;
   }
-  // the bins use the cubes' arrays before the cubes do, and the particle copy
+  // the bins use the rows' arrays before the rows do, and the particle copy
   // that the next reorder overwrites
   float* const other = d_f_[cur_ ^ 1];
   const mpmk::MeshScratch w{d_mcount_, d_moff_, d_mscratch_, other ? (uint32_t*)(other + 3 * stride_) : nullptr,
@@ -665,8 +762,8 @@ int Sim::mesh_build(int side, int radius, int64_t* ntri, hipStream_t s) {
   const double fill = std::min(1.0, (double)std::max<int64_t>(1, occupied_) / (double)node_blocks());
   HIPCHK(mpmk::mesh_distance_field(particles(), side, vdx_f, cutoff, fill, w, d_sdf_, s), "mesh distance field");
   HIPCHK(mpmk::mesh_count(d_sdf_, side, rv, d_mcount_, s), "mesh count");
-  uint32_t* total = d_moff_ + ncubes;
-  HIPCHK(mpmk::exclusive_scan(d_mcount_, d_moff_, (int64_t)ncubes, d_mscratch_, total, s), "mesh scan");
+  uint32_t* total = d_moff_ + rows;
+  HIPCHK(mpmk::exclusive_scan(d_mcount_, d_moff_, (int64_t)rows, d_mscratch_, total, s), "mesh scan");
   uint32_t n = 0;
   HIPCHK(hipMemcpyAsync(&n, total, sizeof(uint32_t), hipMemcpyDeviceToHost, s), "mesh size");
   HIPCHK(hipStreamSynchronize(s), "mesh size");
@@ -692,9 +789,14 @@ int Sim::mesh_triangles(float* xyz, uint64_t* keys) {
   if (mesh_ntri_ < 0) return fail(MPM_ERR_STATE, "mpm_mesh_triangles: no mesh built");
   const size_t n = (size_t)mesh_ntri_;
   if (n == 0) return MPM_OK;
-  if (xyz) HIPCHK(hipMemcpy(xyz, d_mxyz_, sizeof(float) * 9 * n, hipMemcpyDeviceToHost), "mesh triangles");
-  if (keys) HIPCHK(hipMemcpy(keys, d_mkeys_, sizeof(uint64_t) * 3 * n, hipMemcpyDeviceToHost), "mesh edges");
-  return MPM_OK;
+  const auto fetch = [&](void* dst, const void* src, size_t bytes) {
+    return fetch_chunks((const uint8_t*)src, bytes,
+                        [&](size_t off, const uint8_t* data, size_t len) { std::memcpy((uint8_t*)dst + off, data, len); },
+                        nullptr);
+  };
+  int rc = xyz ? fetch(xyz, d_mxyz_, sizeof(float) * 9 * n) : MPM_OK;
+  if (!rc && keys) rc = fetch(keys, d_mkeys_, sizeof(uint64_t) * 3 * n);
+  return rc;
 }
 
 int Sim::mesh_distance(int side, float* out) {
@@ -1162,103 +1264,6 @@ int Sim::advance(int32_t substeps, hipStream_t s) {
     if (rc) return rc;
     t_ += (double)prm_.dt;  // mpm.cu:328
   }
-  return MPM_OK;
-}
-
-// The bytes pass through pinned slots, whose copies run at the link's rate
-// (about 50 GB/s here; straight into pageable memory they run at 10). Taking
-// a chunk out of its slot is the slow part: the caller's arrays are mostly
-// new memory, whose pages the system hands out one fault at a time, at 3 to 5
-// GB/s a thread. So one thread for every 2 MB, up to one a slot, takes
-// chunks, while this one keeps the copies queued on s.
-template <class Take>
-int Sim::fetch_chunks(const uint8_t* src, size_t bytes, const Take& take, hipStream_t s) {
-  if (bytes == 0) return MPM_OK;
-  const size_t cores = std::max(1u, std::thread::hardware_concurrency());
-  size_t slots = std::min({(size_t)kStageSlots, cores, (bytes + ((size_t)2 << 20) - 1) >> 21});
-  const size_t chunk = std::min(kStageBytes, ((bytes + slots - 1) / slots + 4095) & ~(size_t)4095);
-  for (size_t w = 0; w < slots; ++w) {
-    if (stage_bytes_[w] < chunk) {
-      if (h_stage_[w]) (void)hipHostFree(h_stage_[w]);
-      h_stage_[w] = nullptr;
-      stage_bytes_[w] = 0;
-      HIPCHK(hipHostMalloc((void**)&h_stage_[w], chunk, 0), "hipHostMalloc(download)");
-      stage_bytes_[w] = chunk;
-    }
-    if (!stage_ev_[w]) HIPCHK(hipEventCreateWithFlags(&stage_ev_[w], hipEventDisableTiming), "hipEventCreate");
-  }
-  const size_t n = (bytes + chunk - 1) / chunk;
-  const auto size_of = [&](size_t c) { return std::min(chunk, bytes - c * chunk); };
-  const auto queue = [&](size_t c) {
-    const size_t w = c % slots;
-    hipError_t e = hipMemcpyAsync(h_stage_[w], src + c * chunk, size_of(c), hipMemcpyDeviceToHost, s);
-    return e == hipSuccess ? hipEventRecord(stage_ev_[w], s) : e;
-  };
-  std::mutex m;
-  std::condition_variable cv;
-  size_t queued = 0;                       // chunks whose copies are on the stream (under m, as the rest)
-  bool stop = false;
-  std::vector<size_t> taken(slots, 0);     // chunks taken out of each slot
-  std::vector<hipError_t> bad(slots, hipSuccess);
-  // slot w's thread: chunks w, w + slots, ...
-  const auto work = [&](size_t w) {
-    hipError_t e = hipSetDevice(device_);
-    for (size_t c = w; c < n; c += slots) {
-      {
-        std::unique_lock<std::mutex> lock(m);
-        cv.wait(lock, [&] { return queued > c || stop; });
-        if (queued <= c) return;
-      }
-      if (e == hipSuccess) e = hipEventSynchronize(stage_ev_[w]);
-      if (e == hipSuccess) take(c * chunk, h_stage_[w], size_of(c));
-      std::lock_guard<std::mutex> lock(m);
-      ++taken[w];
-      bad[w] = e;
-      cv.notify_all();
-    }
-  };
-  std::vector<std::thread> threads;
-  if (slots > 1) {
-    try {
-      for (size_t w = 0; w < slots; ++w) threads.emplace_back(work, w);
-    } catch (const std::exception&) {
-      // no more threads to be had: those that started end, and one slot does
-      {
-        std::lock_guard<std::mutex> lock(m);
-        stop = true;
-      }
-      cv.notify_all();
-      for (auto& t : threads) t.join();
-      threads.clear();
-      slots = 1;
-    }
-  }
-  hipError_t e = hipSuccess;
-  if (threads.empty()) {
-    for (size_t c = 0; c < n && e == hipSuccess; ++c) {
-      e = queue(c);
-      if (e == hipSuccess) e = hipEventSynchronize(stage_ev_[c % slots]);
-      if (e == hipSuccess) take(c * chunk, h_stage_[c % slots], size_of(c));
-    }
-    HIPCHK(e, "download");
-    return MPM_OK;
-  }
-  for (size_t c = 0; c < n && e == hipSuccess; ++c) {
-    const size_t w = c % slots;
-    {
-      std::unique_lock<std::mutex> lock(m);
-      cv.wait(lock, [&] { return taken[w] == c / slots || bad[w] != hipSuccess; });
-      e = bad[w];
-    }
-    if (e == hipSuccess) e = queue(c);
-    std::lock_guard<std::mutex> lock(m);
-    if (e == hipSuccess) queued = c + 1;
-    else stop = true;
-    cv.notify_all();
-  }
-  for (auto& t : threads) t.join();
-  for (size_t w = 0; w < slots && e == hipSuccess; ++w) e = bad[w];
-  HIPCHK(e, "download");
   return MPM_OK;
 }
 

@@ -207,7 +207,7 @@ class Sim {
   bool dense_ = false;
   int64_t occupied_ = 0;  // home blocks holding particles at the upload
   size_t staged_on_device_ = 0;  // staged particles the last upload / append copied
-  // mesh buffers: distance field, per-cube counts and offsets, scan scratch,
+  // mesh buffers: distance field, per-row counts and offsets (or the bins'), scan scratch,
   // triangles; the last build's grid side and triangle count
   uint32_t* d_sdf_ = nullptr;
   uint32_t* d_mcount_ = nullptr;

@@ -222,9 +222,10 @@ hipError_t tile_combine(const TileSums& in, int64_t nblk, hipStream_t s);
 // mesh.hip: surface mesh of the particles. The distance field (side^3
 // voxels of edge vdx, float bits) starts at `cutoff` and takes the distance
 // to every particle whose box of voxels reaches it; mesh_count writes the
-// triangle count of each of the (side-1)^3 cubes of S = rv - distance = 0,
-// mesh_emit writes them (9 floats each, and the 3 grid edges their
-// vertices lie on) at the scanned offsets.
+// triangle count of each of the (side-1)^2 rows of cubes of S = rv - distance
+// = 0, mesh_emit writes them (9 floats each, and the 3 grid edges their
+// vertices lie on, cube after cube) at the rows' scanned offsets (one more
+// entry than rows: the total).
 // Scratch of the field: mesh_bins(side)^3 counts, one start more, the scan's
 // tile sums (one per 2048 counts), a rank and 3 planes of pos_stride floats
 // for the particles.
