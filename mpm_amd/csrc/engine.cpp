@@ -641,8 +641,9 @@ int Sim::fetch_chunks(const uint8_t* src, size_t bytes, const Take& take, hipStr
       if (h_stage_[w]) (void)hipHostFree(h_stage_[w]);
       h_stage_[w] = nullptr;
       stage_bytes_[w] = 0;
-      HIPCHK(hipHostMalloc((void**)&h_stage_[w], chunk, 0), "hipHostMalloc(download)");
-      stage_bytes_[w] = chunk;
+      const size_t want = slots > 1 ? kStageBytes : chunk;
+      HIPCHK(hipHostMalloc((void**)&h_stage_[w], want, 0), "hipHostMalloc(download)");
+      stage_bytes_[w] = want;
     }
     if (!stage_ev_[w]) HIPCHK(hipEventCreateWithFlags(&stage_ev_[w], hipEventDisableTiming), "hipEventCreate");
   }

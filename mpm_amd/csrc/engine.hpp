@@ -186,7 +186,7 @@ class Sim {
   // pinned slots of fetch_chunks, each with the event of its last copy; at
   // most kStageSlots of kStageBytes a handle
   static constexpr int kStageSlots = 8;
-  static constexpr size_t kStageBytes = (size_t)4 << 20;
+  static constexpr size_t kStageBytes = (size_t)2 << 20;
   uint8_t* h_stage_[kStageSlots] = {};
   size_t stage_bytes_[kStageSlots] = {};
   hipEvent_t stage_ev_[kStageSlots] = {};
