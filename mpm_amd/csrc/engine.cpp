@@ -902,13 +902,10 @@ int Sim::sort_particles(hipStream_t s) {
   const ParticlesDev src = particles();
   int out = 0;
   PHASE(PH_SORT, {
-    HIPCHK(mpmk::cell_keys(src, k_, lb_, d_keys_[0], d_vals_[0], s), "cell keys");
     // by home block only: k_item_arrange orders each item by cell
-    HIPCHK(mpmk::radix_sort(d_keys_, d_vals_, P_, 3 * lb_, mpmk::cell_key_bits(k_.N, lb_),
-                            (int)opt_.radix_bits, d_hist_, &out, s),
-           "radix sort");
+    HIPCHK(mpmk::cell_sort(src, k_, lb_, d_keys_, d_vals_, (int)opt_.radix_bits, d_hist_, &out, s), "cell sort");
     HIPCHK(mpmk::build_items(d_keys_[out], d_vals_[out], P_, lb_, chunk_, nblk_, d_block_start_,
-                             d_block_items_, d_covered_, (k_.N + 3) / 4, d_flag_, d_pos_, d_hist_,
+                             d_block_items_, d_covered_, (k_.N + 3) / 4, d_pos_, d_hist_,
                              d_item_count_, d_item_start_, d_item_block_, d_item_waves_, d_gather_,
                              items, d_crowded_, s),
            "work items");
@@ -945,7 +942,6 @@ int Sim::sort_desc(mpmk::SortDesc& d) {
   d.crowded = d_crowded_;
   d.nblk = nblk_;
   d.nbx = (k_.N + 3) / 4;
-  d.flag = d_flag_;
   d.pos = d_pos_;
   d.item_count = d_item_count_;
   d.item_start = d_item_start_;
@@ -1271,7 +1267,7 @@ int Sim::advance(int32_t substeps, hipStream_t s) {
 // The rows are put in original-index order on the device (k_export) in the
 // particle copy that the next reorder overwrites, then fetched as one range.
 // A pass over the planes on the host took 75 ms for 1,000,000 particles (an
-// id's 25 values from 25 planes), 0.2 ms on the device.
+// id's 25 values from 25 planes); the device takes 0.1 ms and the fetch 3.
 int Sim::download_soa(float* x, float* v, float* C, float* F, float* Jp, uint8_t* mat,
                       hipStream_t s) {
   if (!uploaded_) return fail(MPM_ERR_STATE, "mpm_download_soa: nothing uploaded");

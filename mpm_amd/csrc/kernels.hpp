@@ -33,6 +33,10 @@ hipError_t cell_keys(const ParticlesDev& P, const StepConsts& k, int lb, uint32_
 // holds radix_scratch_words() words.
 hipError_t radix_sort(uint32_t* keys[2], uint32_t* vals[2], int64_t n, int start_bit, int key_bits,
                       int radix_bits, uint32_t* scratch, int* out_idx, hipStream_t s);
+// cell_keys and radix_sort by the bits above the cell within the block, the
+// first histogram made with the keys
+hipError_t cell_sort(const ParticlesDev& P, const StepConsts& k, int lb, uint32_t* keys[2], uint32_t* vals[2],
+                     int radix_bits, uint32_t* scratch, int* out_idx, hipStream_t s);
 hipError_t exclusive_scan(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* scratch,
                           uint32_t* total, hipStream_t s);
 hipError_t fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t s);
@@ -58,7 +62,7 @@ constexpr int kTileNodes = kTileW * kTileW * kTileW;
 // item's tile can reach.
 hipError_t build_items(const uint32_t* keys, const uint32_t* perm, int64_t n, int lb, int chunk,
                        int64_t nblk, uint32_t* block_range, uint32_t* block_items, uint32_t* covered,
-                       int nbx, uint32_t* flag, uint32_t* pos, uint32_t* scratch, uint32_t* total,
+                       int nbx, uint32_t* pos, uint32_t* scratch, uint32_t* total,
                        uint32_t* item_start, uint32_t* item_block, uint32_t* item_waves,
                        uint32_t* gather, int64_t max_items, uint32_t* crowded, hipStream_t s);
 // Removes the particles with original index in [lo, hi): the others packed
@@ -183,7 +187,6 @@ struct SortDesc {
   uint32_t* covered;
   int64_t nblk;
   int nbx;
-  uint32_t* flag;
   uint32_t* pos;
   uint32_t* item_count;
   uint32_t* item_start;
@@ -198,7 +201,7 @@ struct SortDesc {
 // 8-bit pass (pass = 0, 1, ...)
 enum SortPhase : int {
   SORT_FILL = 0, SORT_KEYS, SORT_HIST, SORT_RSCAN, SORT_SCATTER, SORT_HEADS, SORT_FLAGS,
-  SORT_SCAN_TILES, SORT_SCAN_SUMS, SORT_SCAN_ADD, SORT_EMIT, SORT_ARRANGE, SORT_CROWDED, SORT_NUM_PHASES
+  SORT_SCAN_SUMS, SORT_EMIT, SORT_ARRANGE, SORT_NUM_PHASES
 };
 // workgroups of one scene in a phase (0: the scene sits the phase out)
 int64_t sort_blocks(const SortDesc& d, int phase, int pass);
