@@ -10,33 +10,37 @@
 // velocity and mass after the update (N^3 float4, read by G2P), then the
 // velocity before the walls and the wall flags (N^3 float4).
 //
-// Kernels, one particle per lane, one wavefront per workgroup:
+// Kernels, 64 particles and four wavefronts per workgroup (a particle is lane i
+// of each):
 //   k_diff_step<G2P, P2G>   G2P of substep n (gather of the tape velocities,
 //                           F and x update) fused with the P2G of substep n+1
 //                           (stress through the polar rotation of F, scatter)
 //   k_diff_grid             grid update into the tape; clears the grid
 //   k_adj_step<P2G', G2P'>  the adjoint of the P2G of substep s (gather of the
-//                           momentum and mass adjoints, stress adjoint through
-//                           the SVD, mu and lambda adjoints) fused with the
-//                           adjoint of the G2P of substep s-1 (scatter of the
-//                           grid velocity adjoint)
+//                           momentum and mass adjoints, stress adjoint, mu and
+//                           lambda adjoints) fused with the adjoint of the G2P
+//                           of substep s-1 (scatter of the grid velocity
+//                           adjoint)
 //   k_adj_grid              grid update backward: momentum and mass adjoints
 // so a substep is two launches forward and two backward, and a run of
 // substeps is enqueued from one host call (diff_forward_steps /
 // diff_backward_steps).
 //
-// The stress adjoint differentiates the polar rotation R of F = U S V^T:
-// with Rbar the adjoint of R and M = V^T skew(R^T Rbar) V,
-// Fbar += 2 U N V^T, N_ij = M_ij / (s_i + s_j).
+// What bounds them is latency: the elastic cube of 32,768 particles is 512
+// workgroups on 256 CUs, a small one 35, and the state that a substep moves
+// (200 bytes a particle, 6.5 MB) takes 1.3 us at the copy rate. So three
+// wavefronts take an x-plane of the stencil each and run what needs a whole
+// particle (stress, F) side by side, a fourth takes what does not wait for
+// them (storing the state, the cells of the scatter, the SVD of mu's adjoint).
+// A wavefront has its SIMD nearly to itself and runs its code once: short code
+// without branches, in which an LDS or memory round trip is waited for once, is
+// what counts. k_diff_step and k_adj_step took 25 and 38 us for 32,768
+// particles with one wavefront per 64 particles, now 10.2 and 12.6 (2,197
+// particles: 19 and 29, now 7.8 and 9.7).
 //
-// Scatters (P2G: 27 nodes x 4 values; the grid adjoint of G2P: 27 x 3): each
-// lane writes its particle's values into a row of an LDS table; then each
-// lane takes a column and walks the rows in lane order, summing runs -- a run
-// is a stretch of lanes whose particles share a base cell (particles sorted by
-// cell make long runs: ~37 per cell for a dense lattice) -- and adding each
-// run's sum to the grid with one FP32 atomic. A dense scene issues ~3 runs x
-// 108 atomics per wavefront instead of 64 x 108; unsorted particles only give
-// shorter runs.
+// The stress adjoint differentiates the polar rotation R of F = R S: with
+// Rbar the adjoint of R and K = skew(R^T Rbar), Fbar += 2 R X for the skew X
+// with S X + X S = K.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -51,11 +55,12 @@ namespace {
 
 enum : int { DX = 0, DV = 3, DC = 6, DF = 15 };
 
-constexpr int kWave = 64;        // lanes per workgroup (one wavefront)
-constexpr int kP2GVals = 108;    // 27 nodes x (momentum, mass)
-constexpr int kP2GStride = 109;  // odd LDS row stride: a column spreads over the banks
-constexpr int kAdjVals = 81;     // 27 nodes x grid velocity adjoint
-constexpr int kAdjStride = 83;
+constexpr int kWave = 64;            // particles per workgroup
+constexpr int kPlanes = 3;           // wavefronts per workgroup: one per x-plane of the stencil, and a
+constexpr int kThreads = 4 * kWave;  // fourth for what does not wait for the planes
+constexpr int kNodes = 27;           // of a stencil
+constexpr int kRunsAhead = 8;        // runs whose sums are loaded together
+constexpr int kNowhere = 1 << 20;    // a cell that no node is next to
 
 struct DiffK {
   StepConsts k;
@@ -63,10 +68,18 @@ struct DiffK {
   int64_t n;
 };
 
-// quadratic B-spline weights and their derivatives (InterpolationKernel.cuh)
+// One axis of a particle's stencil: quadratic B-spline weights and their
+// derivatives (InterpolationKernel.cuh), node offsets and node indices. A node
+// outside the grid has weight 0 and the index of the nearest node inside,
+// which the stencil of a particle that reaches the grid has anyway.
+struct Axis {
+  int base;
+  int node[3];
+  float w[3], dw[3], dp[3];
+};
+
 struct Stencil {
-  int base[3];
-  float w[3][3], dw[3][3];
+  Axis ax[3];
   bool outside;  // no node of the stencil in the grid: the particle is left as it is
 };
 
@@ -75,94 +88,134 @@ __device__ __forceinline__ Stencil make_stencil(const float x[3], const StepCons
   s.outside = false;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
+    Axis& t = s.ax[a];
     const float xg = x[a] * k.dx_inv;
-    s.base[a] = (int)(xg - 0.5f);
-    const float f = xg - (float)s.base[a];
+    t.base = (int)(xg - 0.5f);
+    const float f = xg - (float)t.base;
     const float t0 = 1.5f - f, t1 = f - 1.0f, t2 = f - 0.5f;
-    s.w[a][0] = 0.5f * (t0 * t0);
-    s.w[a][1] = 0.75f - t1 * t1;
-    s.w[a][2] = 0.5f * (t2 * t2);
-    s.dw[a][0] = -t0 * k.dx_inv;
-    s.dw[a][1] = -2.0f * t1 * k.dx_inv;
-    s.dw[a][2] = t2 * k.dx_inv;
-    s.outside |= s.base[a] + 3 < 0 || s.base[a] >= k.N;  // mpm.cu:31-35,129-133
+    const float w[3] = {0.5f * (t0 * t0), 0.75f - t1 * t1, 0.5f * (t2 * t2)};
+    const float dw[3] = {-t0 * k.dx_inv, -2.0f * t1 * k.dx_inv, t2 * k.dx_inv};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int node = t.base + i;
+      const bool ok = (unsigned)node < (unsigned)k.N;
+      t.w[i] = ok ? w[i] : 0.0f;
+      t.dw[i] = ok ? dw[i] : 0.0f;
+      t.dp[i] = (float)node * k.dx - x[a];
+      t.node[i] = min(max(node, 0), k.N - 1);
+    }
+    s.outside |= t.base + 3 < 0 || t.base >= k.N;  // mpm.cu:31-35,129-133
   }
   return s;
 }
 
-__device__ __forceinline__ bool node_ok(const Stencil& s, int a, int b, int c, int N) {
-  return (unsigned)(s.base[0] + a) < (unsigned)N && (unsigned)(s.base[1] + b) < (unsigned)N &&
-         (unsigned)(s.base[2] + c) < (unsigned)N;
+// the entry of an x-axis array that a wavefront's plane has
+template <typename T>
+__device__ __forceinline__ T of_plane3(T a, T b, T c, int plane) {
+  return plane == 0 ? a : plane == 1 ? b : c;
 }
-
-__device__ __forceinline__ size_t node_index(const Stencil& s, int a, int b, int c, int N) {
-  return ((size_t)(s.base[0] + a) * N + (size_t)(s.base[1] + b)) * N + (size_t)(s.base[2] + c);
-}
-
-__device__ __forceinline__ float weight(const Stencil& s, int a, int b, int c) {
-  return (s.w[0][a] * s.w[1][b]) * s.w[2][c];
-}
-
-__device__ __forceinline__ void weight_grad(const Stencil& s, int a, int b, int c, float gw[3]) {
-  gw[0] = (s.dw[0][a] * s.w[1][b]) * s.w[2][c];
-  gw[1] = (s.w[0][a] * s.dw[1][b]) * s.w[2][c];
-  gw[2] = (s.w[0][a] * s.w[1][b]) * s.dw[2][c];
-}
-
-__device__ __forceinline__ void node_offset(const Stencil& s, int a, int b, int c, const float x[3],
-                                            const StepConsts& k, float dp[3]) {
-  dp[0] = (float)(s.base[0] + a) * k.dx - x[0];
-  dp[1] = (float)(s.base[1] + b) * k.dx - x[1];
-  dp[2] = (float)(s.base[2] + c) * k.dx - x[2];
+template <typename T>
+__device__ __forceinline__ T of_plane(const T (&v)[3], int plane) {
+  return of_plane3(v[0], v[1], v[2], plane);
 }
 
 // the base cell of a particle inside the domain (base in [-3, N) per axis)
 // as one non-negative integer
 __device__ __forceinline__ int cell_key(const Stencil& s, int N) {
   const int M = N + 3;
-  return ((s.base[0] + 3) * M + (s.base[1] + 3)) * M + (s.base[2] + 3);
+  return ((s.ax[0].base + 3) * M + (s.ax[1].base + 3)) * M + (s.ax[2].base + 3);
 }
 
-__device__ __forceinline__ void load_xF(const float* st, int64_t n, int64_t p, float x[3], float F[9]) {
+template <int PLANES>
+__device__ __forceinline__ void load_planes(const float* st, int64_t n, int64_t p, int first, float* out) {
 #pragma unroll
-  for (int a = 0; a < 3; ++a) x[a] = st[(DX + a) * n + p];
-#pragma unroll
-  for (int a = 0; a < 9; ++a) F[a] = st[(DF + a) * n + p];
+  for (int a = 0; a < PLANES; ++a) out[a] = st[(first + a) * n + p];
 }
 
-__device__ __forceinline__ void load_state(const float* st, int64_t n, int64_t p, float x[3],
-                                           float v[3], float C[9], float F[9]) {
+template <int PLANES>
+__device__ __forceinline__ void store_planes(float* st, int64_t n, int64_t p, int first, const float* in) {
 #pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    x[a] = st[(DX + a) * n + p];
-    v[a] = st[(DV + a) * n + p];
-  }
-#pragma unroll
-  for (int a = 0; a < 9; ++a) {
-    C[a] = st[(DC + a) * n + p];
-    F[a] = st[(DF + a) * n + p];
-  }
+  for (int a = 0; a < PLANES; ++a) st[(first + a) * n + p] = in[a];
 }
 
-__device__ __forceinline__ void store_state(float* st, int64_t n, int64_t p, const float x[3],
+// a particle's 24 values, shared out to the three wavefronts that hold them
+__device__ __forceinline__ void store_state(float* st, int64_t n, int64_t p, int plane, const float x[3],
                                             const float v[3], const float C[9], const float F[9]) {
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    st[(DX + a) * n + p] = x[a];
-    st[(DV + a) * n + p] = v[a];
+  if (plane == 0) {
+    store_planes<3>(st, n, p, DX, x);
+    store_planes<3>(st, n, p, DV, v);
+  } else if (plane == 1) {
+    store_planes<9>(st, n, p, DC, C);
+  } else if (plane == 2) {
+    store_planes<9>(st, n, p, DF, F);
   }
+}
+
+// ---------------------------------------------------------------- rotation
+// The SVD for the particles polar_rotation leaves: out of line, so that its
+// registers do not count against the kernels'.
+__device__ __noinline__ void svd_rotation(const float* F, float* R) {
+  float U[9], s[3], V[9];
+  svd3_robust(F, U, s, V);
+  mul_abt(U, V, R);
+}
+
+// The polar rotation R of F = R S. Newton's iteration X <- (X + X^-T) / 2
+// (Higham, "Computing the polar decomposition", 1986) from X = F: with
+// singular values in (1/8, 8) and det F > 0 it converges quadratically to the
+// rotation that U V^T of the SVD is, and its 42 operations a step have nothing
+// serial but the determinant's reciprocal. A solid that is deformed by 1 %
+// takes 3 steps, with the stress 0.6 us (1,500 cycles) of a wavefront that has
+// its SIMD to itself, where the Jacobi SVD's chain of 12 rotations, sort and QR
+// is 870 instructions, over 2 us. The other particles (turned inside out,
+// crushed or drawn out, not finite) go through the SVD; returns whether this
+// lane's did. Every lane of the wavefront calls it.
+__device__ __forceinline__ bool polar_rotation(const float F[9], bool live, float R[9]) {
+  float X[9];
 #pragma unroll
-  for (int a = 0; a < 9; ++a) {
-    st[(DC + a) * n + p] = C[a];
-    st[(DF + a) * n + p] = F[a];
+  for (int i = 0; i < 9; ++i) X[i] = F[i];
+  bool bad = false, done = !live;
+  for (int it = 0; it < 8; ++it) {
+    const float cof[9] = {X[4] * X[8] - X[5] * X[7], X[5] * X[6] - X[3] * X[8], X[3] * X[7] - X[4] * X[6],
+                          X[2] * X[7] - X[1] * X[8], X[0] * X[8] - X[2] * X[6], X[1] * X[6] - X[0] * X[7],
+                          X[1] * X[5] - X[2] * X[4], X[2] * X[3] - X[0] * X[5], X[0] * X[4] - X[1] * X[3]};
+    const float det = X[0] * cof[0] + X[1] * cof[1] + X[2] * cof[2];
+    const float h = 0.5f / det;
+    float step = 0.0f, size = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+      const float y = __builtin_fmaf(h, cof[i], 0.5f * X[i]);
+      const float dx = y - X[i];
+      step += dx * dx;
+      size += y * y;
+      X[i] = y;
+    }
+    // after one step a singular value s has become (s + 1/s) / 2: above 4.06
+    // for s past 8 or 1/8
+    if (it == 0) bad = !(det > 0.0f) || !(size < 16.5f);
+    // (the step's length is the error before it, half its square the one after)
+    done |= bad || step < 1e-7f;
+    if (__ballot(!done) == 0ull) break;
   }
+  bad = live && (bad || !done);
+#pragma unroll
+  for (int i = 0; i < 9; ++i) R[i] = X[i];
+  if (bad) {
+    // (the copies are the arrays whose address the call takes: F and R of the
+    // common path stay in registers)
+    float f[9], r[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) f[i] = F[i];
+    svd_rotation(f, r);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) R[i] = r[i];
+  }
+  return bad;
 }
 
 // tau = 2 mu (F - R) F^T + lambda (J - 1) J I, J = det F
-__device__ __forceinline__ void fc_stress(const float F[9], float mu, float lam, float U[9],
-                                          float s[3], float V[9], float R[9], float tau[9]) {
-  svd3_robust(F, U, s, V);
-  mul_abt(U, V, R);
+__device__ __forceinline__ void fc_stress(const float F[9], const float R[9], float mu, float lam,
+                                          float tau[9]) {
   float FmR[9];
 #pragma unroll
   for (int i = 0; i < 9; ++i) FmR[i] = 2.0f * mu * (F[i] - R[i]);
@@ -179,81 +232,318 @@ __device__ __forceinline__ float stress_scale(const DiffK& d) {
   return ((-d.k.dinv) * d.k.dt) * d.volume;
 }
 
-// ---------------------------------------------------------------- run scatter
-// Adds the LDS table rows (NV values per lane, row stride STRIDE; VPN values
-// per node, stencil node o = 9a + 3b + c at columns VPN o .. VPN o + VPN - 1)
-// to `grid` (4 floats per node): one sum per (run, column), in lane order,
-// and one FP32 atomic per non-zero sum of a node inside the grid. A run is a
-// stretch of lanes with the same key (key < 0: the lane adds nothing). Each
-// lane takes a column and walks the rows in lane order, 16 rows loaded at a
-// time; the run ends are the same for every column, so the walk branches
-// uniformly and a run's atomics for 64 columns are one instruction. Every
-// lane of the (one-wavefront) workgroup calls it.
-template <int NV, int STRIDE, int VPN>
-__device__ __forceinline__ void run_scatter(const float* table, int key, const int base[3], int N,
-                                            float* __restrict__ grid) {
-  const int lane = threadIdx.x;
-  const int next = __shfl_down(key, 1);
-  const uint64_t ends = __ballot(lane == kWave - 1 || key != next);
-  const uint64_t live = __ballot(key >= 0);
-  __syncthreads();  // the table rows are visible to every lane
-  for (int c0 = 0; c0 < NV; c0 += kWave) {
-    const int q = c0 + lane;
-    const bool qok = q < NV;
-    const int qc = qok ? q : 0;  // (a column past the table reads column 0, unused)
-    const int o = qc / VPN, comp = qc - (qc / VPN) * VPN;
-    const int da = o / 9, db = (o / 3) % 3, dc = o % 3;
-    float sum = 0.0f;
+// ---------------------------------------------------------------- plane of a stencil
+// One x-plane (9 nodes) of a particle's stencil, as tensor products of the y
+// and z axes: each of the sums over the nodes is taken over z, then over y, so
+// a node costs 6 (velocity and its first moments), 15 (with the gradient) or 8
+// (a row) multiply-adds where the node by node form had 30 to 60.
+
+// the q-vector q0 + M dp of the plane's nodes: at (plane, b) and at node c
+__device__ __forceinline__ void q_start(const float q0[3], const float M[9], float dpa, float qa[3]) {
 #pragma unroll
-    for (int p0 = 0; p0 < kWave; p0 += 16) {
-      float v[16];
+  for (int r = 0; r < 3; ++r) qa[r] = __builtin_fmaf(M[3 * r], dpa, q0[r]);
+}
+
+// Sums over the plane of the 4-vectors g = grid[node]:
+//   s[0..2]    sum w g              s[3 + 3 r + q]  sum w g_r dp_q
+// and with GRAD, val = g . (q0 + M dp) + m g.w (m = 0 without MASS),
+//   s[12 + q]  sum (dw/dx_q) val
+// With ROWS the plane's rows w (q0 + M dp) go to `row`.
+template <bool GRAD, bool MASS, bool ROWS>
+__device__ __forceinline__ void plane_sums(const float4* __restrict__ grid, const Stencil& sn, int plane, int N,
+                                           const float q0[3], const float M[9], float m, float4* row,
+                                           float s[16]) {
+  const Axis &ay = sn.ax[1], &az = sn.ax[2];
+  const float wa = of_plane(sn.ax[0].w, plane), dpa = of_plane(sn.ax[0].dp, plane);
+  const int na = of_plane(sn.ax[0].node, plane);
+  float4 g[9];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) v[i] = table[(p0 + i) * STRIDE + qc];
+  for (int b = 0; b < 3; ++b)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int p = p0 + i;
-        if ((live >> p) & 1ull) sum += v[i];  // (a row of no particle is never read)
-        if ((ends >> p) & 1ull) {
-          if (((live >> p) & 1ull) && qok && sum != 0.0f) {
-            const int gi = __builtin_amdgcn_readlane(base[0], p) + da;
-            const int gj = __builtin_amdgcn_readlane(base[1], p) + db;
-            const int gk = __builtin_amdgcn_readlane(base[2], p) + dc;
-            if ((unsigned)gi < (unsigned)N && (unsigned)gj < (unsigned)N && (unsigned)gk < (unsigned)N)
-              unsafeAtomicAdd(grid + 4 * (((size_t)gi * N + (size_t)gj) * N + (size_t)gk) + comp, sum);
-          }
-          sum = 0.0f;
+    for (int c = 0; c < 3; ++c)
+      g[3 * b + c] = grid[((size_t)na * N + (size_t)ay.node[b]) * N + (size_t)az.node[c]];
+  float qa[3];
+  if (GRAD) q_start(q0, M, dpa, qa);
+  float S0[3] = {0.f, 0.f, 0.f}, S1[3] = {0.f, 0.f, 0.f}, S2[3] = {0.f, 0.f, 0.f};
+  float u0 = 0.f, u1 = 0.f, u2 = 0.f;
+#pragma unroll
+  for (int b = 0; b < 3; ++b) {
+    float T0[3] = {0.f, 0.f, 0.f}, T2[3] = {0.f, 0.f, 0.f}, t0 = 0.f, t2 = 0.f;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const float4 gc = g[3 * b + c];
+      const float gv[3] = {gc.x, gc.y, gc.z};
+      const float wc = az.w[c], wd = az.w[c] * az.dp[c];
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        T0[r] += wc * gv[r];
+        T2[r] += wd * gv[r];
+      }
+      if (GRAD) {
+        float q[3], val = MASS ? m * gc.w : 0.0f;
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+          q[r] = qa[r] + M[3 * r + 1] * ay.dp[b] + M[3 * r + 2] * az.dp[c];
+          val += gv[r] * q[r];
+        }
+        t0 += wc * val;
+        t2 += az.dw[c] * val;
+        if (ROWS) {
+          const float wt = (wa * ay.w[b]) * wc;
+          row[3 * b + c] = make_float4(wt * q[0], wt * q[1], wt * q[2], 0.0f);
         }
       }
     }
+    const float wb = ay.w[b], wbd = ay.w[b] * ay.dp[b];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      S0[r] += wb * T0[r];
+      S1[r] += wbd * T0[r];
+      S2[r] += wb * T2[r];
+    }
+    if (GRAD) {
+      u0 += wb * t0;
+      u1 += ay.dw[b] * t0;
+      u2 += wb * t2;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    s[r] = wa * S0[r];
+    s[3 + 3 * r] = (wa * dpa) * S0[r];
+    s[3 + 3 * r + 1] = wa * S1[r];
+    s[3 + 3 * r + 2] = wa * S2[r];
+  }
+  s[12] = GRAD ? of_plane(sn.ax[0].dw, plane) * u0 : 0.f;
+  s[13] = GRAD ? wa * u1 : 0.f;
+  s[14] = GRAD ? wa * u2 : 0.f;
+  s[15] = 0.f;
+}
+
+// Adds up the planes' parts of the first 4 V4 values of s, in the planes'
+// order: every wavefront of the workgroup ends with the same bits. put_plane
+// by the planes' wavefronts, a barrier, sum_planes by all. `part` has
+// 3 V4 kWave float4.
+template <int V4>
+__device__ __forceinline__ void put_plane(float4* part, int plane, int lane, const float s[16]) {
+#pragma unroll
+  for (int j = 0; j < V4; ++j)
+    part[(plane * V4 + j) * kWave + lane] = make_float4(s[4 * j], s[4 * j + 1], s[4 * j + 2], s[4 * j + 3]);
+}
+template <int V4>
+__device__ __forceinline__ void sum_planes(const float4* part, int lane, float s[16]) {
+#pragma unroll
+  for (int j = 0; j < V4; ++j) {
+    const float4 a = part[j * kWave + lane], b = part[(V4 + j) * kWave + lane],
+                 c = part[(2 * V4 + j) * kWave + lane];
+    s[4 * j] = (a.x + b.x) + c.x;
+    s[4 * j + 1] = (a.y + b.y) + c.y;
+    s[4 * j + 2] = (a.z + b.z) + c.z;
+    s[4 * j + 3] = (a.w + b.w) + c.w;
   }
 }
 
-// v' = sum_i w_i v_i and C' = Dinv sum_i w_i v_i (x_i - x_p)^T over the stencil
-__device__ __forceinline__ void g2p_affine(const Stencil& sn, const float x[3], const float4* vel,
-                                           const StepConsts& k, float vn[3], float Cn[9]) {
+// ---------------------------------------------------------------- scatter
+// largest value over the wavefront's lanes (v >= 0), the same in every lane
+__device__ __forceinline__ int wave_max(int v) { return __builtin_amdgcn_readlane(wave_max_scan(v), kWave - 1); }
+
+// What the wavefronts of a scatter share in LDS.
+struct ScatterShared {
+  float4 rows[kWave * kNodes + kWave];  // a run's 27 node sums, and a zero for each lane
+  int4 cell[kWave];                     // a run's base cell, and packed, its place in the box
+  int lo[3], hi[3];                     // box of the base cells
+  int runs;
+  float4 sum[kThreads];                 // a wavefront's nodes on their way to the grid
+  int node[kThreads];
+};
+
+// Adds a workgroup's rows (VPN values for each of the 27 nodes of each of 64
+// particles) to `grid` (4 floats per node). Many workgroups aim at the same
+// few nodes, so the rows are summed twice before the FP32 atomics:
+//   scatter_runs   each plane's wavefront sums its 9 nodes over the runs of
+//                  particles of one cell (cut every 16 lanes), a segmented
+//                  scan over the lanes in registers, and puts the runs' sums
+//                  into LDS
+//   scatter_nodes  after a barrier, a lane takes a node of the box that the
+//                  workgroup's particles reach, adds up the runs that touch it
+//                  and sends the sum to `grid`
+// 32,768 particles at 25 a cell have 4 runs in a workgroup at the start of a
+// rollout and 19 (of 8 cells) after 100 substeps, and reach 54 and 82 nodes,
+// where an atomic per run and node makes 100 and 520: 100 substeps take 2.86
+// ms with the runs' atomics alone and 1.72 summed by node. Tried besides: a
+// walk over the 64 rows (50 cycles a row unrolled, 200 in a loop: 5 us and
+// more), and LDS atomics into the box, run by run (a wavefront's 64 lanes take
+// 130 cycles or more per instruction: 14.9 us for the kernel, this 12.6).
+// A box of more nodes than the workgroup has threads (particles in no order,
+// or from the end of one row of cells and the start of the next) goes run by
+// run to `grid`: a second pass over the runs costs more than the atomics saved
+// (4,096 particles in rows of the lattice: a substep and its adjoint 49 us
+// with up to 384 nodes, 43 with one pass; 32,768 in order: no difference).
+//
+// A lane's place among the runs; `inside`: its particle reaches the grid (the
+// same in every wavefront). Every lane of the wavefront calls it.
+struct Runs {
+  uint64_t ends;  // the last lane of each run
+  int depth;      // lanes of the run before this one
+  int run;        // its number
+};
+__device__ __forceinline__ Runs find_runs(bool inside, const Stencil& sn, int N) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int key = inside ? cell_key(sn, N) : -1;
+  const int prev = __shfl_up(key, 1);
+  const uint64_t starts = __ballot((lane & 15) == 0 || key != prev);
+  Runs r;
+  r.ends = (starts >> 1) | (1ull << 63);
+  r.depth = lane - (63 - __clzll((long long)(starts & ((2ull << lane) - 1ull))));
+  r.run = (int)__popcll(r.ends & ((1ull << lane) - 1ull));
+  return r;
+}
+
+// by the planes' wavefronts, all lanes
+template <int VPN>
+__device__ __forceinline__ void scatter_runs(ScatterShared& sh, float4 row[9], bool inside, const Stencil& sn,
+                                             int plane, int N) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const Runs runs = find_runs(inside, sn, N);
+  const int depth = runs.depth;
+  float* v = &row[0].x;
+  // lane i adds lane i - n of its run (a DPP shift within 16 lanes); the mask
+  // drops what belongs to another run, whatever it is
+#define MPM_RUN_STEP(n)                                                                              \
+  {                                                                                                  \
+    int keep = depth >= n ? -1 : 0;                                                                  \
+    __asm__("" : "+v"(keep)); /* (a mask, not a select: one instruction with the shift) */           \
+    _Pragma("unroll") for (int i = 0; i < 36; ++i) if (VPN == 4 || (i & 3) != 3) {                   \
+      const int t = __builtin_amdgcn_update_dpp(0, __float_as_int(v[i]), 0x110 + n, 0xf, 0xf, true); \
+      v[i] += __int_as_float(t & keep);                                                              \
+    }                                                                                                \
+  }
+  MPM_RUN_STEP(1)
+  MPM_RUN_STEP(2)
+  MPM_RUN_STEP(4)
+  MPM_RUN_STEP(8)
+#undef MPM_RUN_STEP
+  if ((runs.ends >> lane) & 1ull) {
 #pragma unroll
-  for (int a = 0; a < 3; ++a) vn[a] = 0.f;
+    for (int o = 0; o < 9; ++o) sh.rows[runs.run * kNodes + 9 * plane + o] = row[o];
+  }
+}
+
+// by the fourth wavefront, all lanes: the runs' cells and the box of nodes they reach
+__device__ __forceinline__ void scatter_cells(ScatterShared& sh, bool inside, const Stencil& sn, int N) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const Runs runs = find_runs(inside, sn, N);
+  const int count = (int)__popcll(runs.ends);
+  int lo[3];
 #pragma unroll
-  for (int i = 0; i < 9; ++i) Cn[i] = 0.f;
+  for (int a = 0; a < 3; ++a) {  // (no particle inside: lo = N, hi = -3)
+    const int base = sn.ax[a].base;
+    const int hi = wave_max(inside ? base + 3 : 0) - 3;
+    lo[a] = N - wave_max(inside ? N - base : 0);
+    if (lane == 0) {
+      sh.lo[a] = lo[a];
+      sh.hi[a] = hi;
+    }
+  }
+  if ((runs.ends >> lane) & 1ull) {
+    const int b0 = sn.ax[0].base, b1 = sn.ax[1].base, b2 = sn.ax[2].base;
+    // (in a box that is summed by node the offsets are below 2^8)
+    sh.cell[runs.run] = inside ? make_int4(b0, b1, b2, (b0 - lo[0]) | (b1 - lo[1]) << 10 | (b2 - lo[2]) << 20)
+                               : make_int4(kNowhere, 0, 0, 0x3fffffff);
+  }
+  sh.rows[kWave * kNodes + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (lane == 0) sh.runs = count;
+}
+
+// Adds component lane & 3 of node lane >> 2 of 16 nodes with one instruction:
+// atomics that lie side by side go out together (a component of 64 nodes at a
+// time, a node's four 16 bytes apart in turn, took 4 times as long).
+__device__ __forceinline__ void add_component(float* __restrict__ grid, int node, int comp, float sum) {
+  if (node >= 0 && sum != 0.0f) unsafeAtomicAdd(grid + 4 * (size_t)(unsigned)node + comp, sum);
+}
+
+// the index of a node of the grid (N <= 1024: below 2^30), -1 outside
+__device__ __forceinline__ int node_index(int i, int j, int k, int N) {
+  return ((unsigned)i < (unsigned)N) & ((unsigned)j < (unsigned)N) & ((unsigned)k < (unsigned)N)
+             ? (i * N + j) * N + k
+             : -1;
+}
+
+// by all wavefronts, a barrier after the two above
+template <int VPN>
+__device__ __forceinline__ void scatter_nodes(ScatterShared& sh, int wave, int N, float* __restrict__ grid) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int runs = __builtin_amdgcn_readfirstlane(sh.runs);
+  const int lo0 = sh.lo[0], lo1 = sh.lo[1], lo2 = sh.lo[2];
+  const int e0 = sh.hi[0] - lo0 + 3, e1 = sh.hi[1] - lo1 + 3, e2 = sh.hi[2] - lo2 + 3;  // nodes per axis
+  if (e0 <= 0) return;
+  // (N <= 1024, so two extents' product is below 2^21)
+  if (e0 * e1 <= kThreads && e0 * e1 * e2 <= kThreads) {
+    const int count = __builtin_amdgcn_readfirstlane(e0 * e1 * e2);
+    const float r1 = __builtin_amdgcn_rcpf((float)e1), r2 = __builtin_amdgcn_rcpf((float)e2);
+    if (wave * kWave < count) {
+      const int node = threadIdx.x;
+      const int ij = (int)(((float)node + 0.5f) * r2);  // (exact: node < 2^8)
+      const int i = (int)(((float)ij + 0.5f) * r1);
+      const int j = ij - i * e1, k = node - ij * e2;
+      const int cells = sh.cell[lane].w;  // run r's, in lane r
+      float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 1
+      for (int r = 0; r < runs; r += kRunsAhead) {
+        float4 v[kRunsAhead];
 #pragma unroll
-  for (int a = 0; a < 3; ++a)
+        for (int q = 0; q < kRunsAhead; ++q) {
+          const int cell = __builtin_amdgcn_readlane(cells, (r + q) & (kWave - 1));
+          const int a = i - (cell & 0x3ff), b = j - ((cell >> 10) & 0x3ff), c = k - (cell >> 20);
+          const bool mine = (max(max((unsigned)a, (unsigned)b), (unsigned)c) < 3u) & (r + q < runs);
+          int at = (r + q) * kNodes + 9 * a + 3 * b + c;
+          at = mine ? at : kWave * kNodes + lane;
+          v[q] = sh.rows[at];
+        }
 #pragma unroll
-    for (int b = 0; b < 3; ++b)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        if (!node_ok(sn, a, b, c, k.N)) continue;
-        const float wt = weight(sn, a, b, c);
-        const float4 gv = vel[node_index(sn, a, b, c, k.N)];
-        float dp[3];
-        node_offset(sn, a, b, c, x, k, dp);
-        const float g[3] = {gv.x, gv.y, gv.z};
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-          vn[r] += wt * g[r];
-#pragma unroll
-          for (int q = 0; q < 3; ++q) Cn[3 * r + q] += (k.dinv * wt) * g[r] * dp[q];
+        for (int q = 0; q < kRunsAhead; ++q) {
+          sum.x += v[q].x;
+          sum.y += v[q].y;
+          sum.z += v[q].z;
+          if (VPN == 4) sum.w += v[q].w;
         }
       }
+      // (the wavefront's own: its LDS accesses are in order)
+      sh.sum[threadIdx.x] = sum;
+      sh.node[threadIdx.x] = node < count ? node_index(lo0 + i, lo1 + j, lo2 + k, N) : -1;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int at = wave * kWave + 16 * q + (lane >> 2), comp = lane & 3;
+        const float part = (&sh.sum[at].x)[comp];
+        if (VPN == 4 || comp != 3) add_component(grid, sh.node[at], comp, part);
+      }
+    }
+  } else {
+    // a thread keeps its node and component, of every other run
+    constexpr int kValues = 4 * kNodes;
+    if (threadIdx.x >= 2 * kValues) return;
+    const int comp = lane & 3, part = threadIdx.x / kValues, o = (threadIdx.x - part * kValues) >> 2;
+    if (VPN == 3 && comp == 3) return;
+    const int a = o / 9, b = (o / 3) % 3, c = o % 3;
+#pragma unroll 1
+    for (int r = part; r < runs; r += 8) {
+      int4 cell[4];
+      float sum[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int at = min(r + 2 * q, runs - 1);
+        cell[q] = sh.cell[at];
+        sum[q] = (&sh.rows[at * kNodes + o].x)[comp];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (r + 2 * q < runs)  // (a cell of kNowhere is outside the grid)
+          add_component(grid, node_index(cell[q].x + a, cell[q].y + b, cell[q].z + c, N), comp, sum[q]);
+    }
+  }
 }
 
 // ---------------------------------------------------------------- forward
@@ -262,75 +552,101 @@ __device__ __forceinline__ void g2p_affine(const Stencil& sn, const float x[3], 
 // of the new state into `grid`. Without G2P: the P2G of `st`. Without P2G:
 // the G2P only.
 template <bool G2P, bool P2G>
-__global__ void __launch_bounds__(kWave)
+__global__ void __launch_bounds__(kThreads)
     k_diff_step(const float* __restrict__ st, float* __restrict__ out, const float4* __restrict__ vel,
                 const float* __restrict__ mu, const float* __restrict__ lam, DiffK d,
                 float* __restrict__ grid) {
-  __shared__ float table[P2G ? kWave * kP2GStride : 1];
-  const int lane = threadIdx.x;
-  const int64_t p = (int64_t)blockIdx.x * kWave + lane;
+  __shared__ float4 part[G2P ? kPlanes * 3 * kWave : 1];
+  __shared__ ScatterShared sh;  // (unused without P2G, then it takes no LDS)
+  const int lane = threadIdx.x & (kWave - 1);
+  const int plane = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t p = (int64_t)blockIdx.x * kWave + lane, n = d.n;
   const StepConsts& k = d.k;
-  const bool valid = p < d.n;
+  const bool valid = p < n;
   float x[3] = {0.f, 0.f, 0.f}, v[3] = {0.f, 0.f, 0.f}, C[9], F[9];
-  Stencil sn;
-  sn.base[0] = sn.base[1] = sn.base[2] = 0;
-  bool inside = false;
+#pragma unroll
+  for (int i = 0; i < 9; ++i) C[i] = F[i] = 0.f;
+  float mup = 0.f, lamp = 0.f;
   if (valid) {
-    load_state(st, d.n, p, x, v, C, F);
-    sn = make_stencil(x, k);
-    inside = !sn.outside;
+    load_planes<3>(st, n, p, DX, x);
+    load_planes<9>(st, n, p, DF, F);
+    if (P2G) {
+      mup = mu[p];
+      lamp = lam[p];
+    }
+    if (!G2P) {
+      load_planes<3>(st, n, p, DV, v);
+      load_planes<9>(st, n, p, DC, C);
+    }
   }
+  Stencil sn = make_stencil(x, k);
+  bool inside = valid && !sn.outside;
   if (G2P) {
+    float s[16];
+    if (plane < kPlanes) {
+      plane_sums<false, false, false>(vel, sn, plane, k.N, nullptr, nullptr, 0.f, nullptr, s);
+      put_plane<3>(part, plane, lane, s);
+    }
+    __syncthreads();
+    sum_planes<3>(part, lane, s);
     if (inside) {
-      float vn[3], Cn[9];
-      g2p_affine(sn, x, vel, k, vn, Cn);
       float A[9];
 #pragma unroll
-      for (int i = 0; i < 9; ++i) A[i] = ((i % 4 == 0) ? 1.0f : 0.0f) + k.dt * Cn[i];
+      for (int i = 0; i < 9; ++i) {
+        C[i] = k.dinv * s[3 + i];
+        A[i] = ((i % 4 == 0) ? 1.0f : 0.0f) + k.dt * C[i];
+      }
       mul_ab(A, F, F);
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        v[a] = vn[a];
-        x[a] = x[a] + k.dt * vn[a];
+        v[a] = s[a];
+        x[a] = x[a] + k.dt * s[a];
       }
-#pragma unroll
-      for (int i = 0; i < 9; ++i) C[i] = Cn[i];
+    } else if (valid) {
+      load_planes<3>(st, n, p, DV, v);
+      load_planes<9>(st, n, p, DC, C);
     }
-    if (valid) store_state(out, d.n, p, x, v, C, F);
-    if (P2G && valid) {
+    if (valid && plane == kPlanes) {
+      store_planes<3>(out, n, p, DX, x);
+      store_planes<3>(out, n, p, DV, v);
+      store_planes<9>(out, n, p, DC, C);
+      store_planes<9>(out, n, p, DF, F);
+    }
+    if (P2G) {
       sn = make_stencil(x, k);
-      inside = !sn.outside;
+      inside = valid && !sn.outside;
     }
   }
-  if (P2G) {
-    int key = -1;
-    if (inside) {
-      float U[9], s[3], V[9], R[9], tau[9];
-      fc_stress(F, mu[p], lam[p], U, s, V, R, tau);
-      const float sc = stress_scale(d);
-      float A[9];
+  if (!P2G) return;
+  if (plane == kPlanes) {
+    scatter_cells(sh, inside, sn, k.N);
+  } else {
+    float R[9], tau[9], A[9];
+    polar_rotation(F, inside, R);
+    fc_stress(F, R, mup, lamp, tau);
+    const float sc = stress_scale(d);
+    float q0[3], qa[3];
 #pragma unroll
-      for (int i = 0; i < 9; ++i) A[i] = sc * tau[i] + d.mass * C[i];
-      float* row = table + lane * kP2GStride;
+    for (int i = 0; i < 9; ++i) A[i] = sc * tau[i] + d.mass * C[i];
 #pragma unroll
-      for (int a = 0; a < 3; ++a)
+    for (int r = 0; r < 3; ++r) q0[r] = d.mass * v[r];
+    q_start(q0, A, of_plane(sn.ax[0].dp, plane), qa);
+    const float wa = of_plane(sn.ax[0].w, plane);
+    float4 row[9];
 #pragma unroll
-        for (int b = 0; b < 3; ++b)
+    for (int b = 0; b < 3; ++b)
 #pragma unroll
-          for (int c = 0; c < 3; ++c) {
-            const int o = 4 * (9 * a + 3 * b + c);
-            const float wt = weight(sn, a, b, c);
-            float dp[3];
-            node_offset(sn, a, b, c, x, k, dp);
+      for (int c = 0; c < 3; ++c) {
+        const float wt = (wa * sn.ax[1].w[b]) * sn.ax[2].w[c];
+        float q[3];
 #pragma unroll
-            for (int r = 0; r < 3; ++r)
-              row[o + r] = wt * (d.mass * v[r] + (A[3 * r] * dp[0] + A[3 * r + 1] * dp[1] + A[3 * r + 2] * dp[2]));
-            row[o + 3] = wt * d.mass;
-          }
-      key = cell_key(sn, k.N);
-    }
-    run_scatter<kP2GVals, kP2GStride, 4>(table, key, sn.base, k.N, grid);
+        for (int r = 0; r < 3; ++r) q[r] = qa[r] + A[3 * r + 1] * sn.ax[1].dp[b] + A[3 * r + 2] * sn.ax[2].dp[c];
+        row[3 * b + c] = make_float4(wt * q[0], wt * q[1], wt * q[2], wt * d.mass);
+      }
+    scatter_runs<4>(sh, row, inside, sn, plane, k.N);
   }
+  __syncthreads();
+  scatter_nodes<4>(sh, plane, k.N, grid);
 }
 
 // grid update into the tape: tv = (velocity, mass) after the update, tw =
@@ -363,6 +679,25 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---------------------------------------------------------------- backward
+// The part of the adjoint of F that comes through its rotation: 2 U N V^T,
+// N_ij = (V^T Sk V)_ij / (s_i + s_j), for the particles whose rotation came
+// from the SVD.
+__device__ __noinline__ void svd_rotation_adjoint(const float* F, const float* Sk, float* out) {
+  float U[9], s[3], V[9], T1[9], Nm[9], UN[9];
+  svd3_robust(F, U, s, V);
+  mul_ab(Sk, V, T1);
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const float mt = V[r] * T1[c] + V[3 + r] * T1[3 + c] + V[6 + r] * T1[6 + c];
+      const float den = s[r] + s[c];
+      Nm[3 * r + c] = (r == c || den == 0.0f) ? 0.0f : 2.0f * mt / den;
+    }
+  mul_ab(U, Nm, UN);
+  mul_abt(UN, V, out);
+}
+
 // The adjoint of the P2G of substep s (P2GA: the momentum and mass adjoints
 // `gm` of that substep, gathered) fused with the adjoint of the G2P of
 // substep s-1 (G2PA: the grid velocity adjoint scattered into `gv_out`).
@@ -373,83 +708,107 @@ __global__ void __launch_bounds__(256)
 //             otherwise the full adjoint of X_s.
 // X_s = st_s (state before substep s), X_{s-1} = st_prev with tape velocities
 // vel_prev. The mu and lambda adjoints are added into adj_mu, adj_lam.
+//
+// The fourth wavefront takes the mu and lambda adjoints off the others:
+// mu's is (F - R) F^T : tb, and F - R of a solid deformed by 1 % turns an
+// error of R into one a hundred times larger, so its R stays the SVD's, whose
+// chain the wavefront runs while the planes gather.
 template <bool P2GA, bool G2PA>
-__global__ void __launch_bounds__(kWave)
+__global__ void __launch_bounds__(kThreads)
     k_adj_step(const float* __restrict__ st_s, const float* __restrict__ mu, const float* __restrict__ lam,
                const float4* __restrict__ gm, const float* adj_src, const float* __restrict__ st_prev,
                const float4* __restrict__ vel_prev, float* adj_dst, float* __restrict__ adj_mu,
                float* __restrict__ adj_lam, float* __restrict__ gv_out, DiffK d) {
-  __shared__ float table[G2PA ? kWave * kAdjStride : 1];
-  const int lane = threadIdx.x;
-  const int64_t p = (int64_t)blockIdx.x * kWave + lane;
+  __shared__ float4 part_p[P2GA ? kPlanes * 4 * kWave : 1];
+  __shared__ float4 part_g[G2PA ? kPlanes * 4 * kWave : 1];
+  __shared__ ScatterShared sh;  // (unused without G2PA)
+  const int lane = threadIdx.x & (kWave - 1);
+  const int plane = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t p = (int64_t)blockIdx.x * kWave + lane, n = d.n;
   const StepConsts& k = d.k;
-  const int64_t n = d.n;
   const bool valid = p < n;
   // adjoint of X_s
   float xb[3] = {0.f, 0.f, 0.f}, vb[3] = {0.f, 0.f, 0.f}, Cb[9], Fb[9];
+  float xp[3] = {0.f, 0.f, 0.f}, Fp[9];  // of X_{s-1}
 #pragma unroll
-  for (int i = 0; i < 9; ++i) Cb[i] = Fb[i] = 0.f;
-  if (valid) load_state(adj_src, n, p, xb, vb, Cb, Fb);
+  for (int i = 0; i < 9; ++i) Cb[i] = Fb[i] = Fp[i] = 0.f;
+  if (valid) {
+    load_planes<3>(adj_src, n, p, DX, xb);
+    load_planes<9>(adj_src, n, p, DF, Fb);
+    if (!P2GA) {
+      load_planes<3>(adj_src, n, p, DV, vb);
+      load_planes<9>(adj_src, n, p, DC, Cb);
+    }
+    if (G2PA) {
+      load_planes<3>(st_prev, n, p, DX, xp);
+      load_planes<9>(st_prev, n, p, DF, Fp);
+    }
+  }
 
-  if (P2GA && valid) {
-    float x[3], v[3], C[9], F[9];
-    load_state(st_s, n, p, x, v, C, F);
+  if (P2GA) {
+    float x[3] = {0.f, 0.f, 0.f}, v[3] = {0.f, 0.f, 0.f}, C[9], F[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) C[i] = F[i] = 0.f;
+    float mup = 0.f, lamp = 0.f;
+    if (valid) {
+      load_planes<3>(st_s, n, p, DX, x);
+      load_planes<9>(st_s, n, p, DF, F);
+      load_planes<3>(st_s, n, p, DV, v);
+      load_planes<9>(st_s, n, p, DC, C);
+      mup = mu[p];
+      lamp = lam[p];
+    }
     const Stencil sn = make_stencil(x, k);
-    if (!sn.outside) {  // outside: the partial already holds the identity map
-      const float mup = mu[p], lamp = lam[p];
-      float U[9], s[3], V[9], R[9], tau[9];
-      fc_stress(F, mup, lamp, U, s, V, R, tau);
-      const float sc = stress_scale(d);
-      float A[9];
+    const bool inside = valid && !sn.outside;
+    float R[9], tau[9], A[9], q0[3];
+    bool by_svd = false;
+    const float sc = stress_scale(d);
+    float s[16];
+    if (plane < kPlanes) {
+      by_svd = polar_rotation(F, inside, R);
+      fc_stress(F, R, mup, lamp, tau);
 #pragma unroll
       for (int i = 0; i < 9; ++i) A[i] = sc * tau[i] + d.mass * C[i];
-      float Ab[9];
 #pragma unroll
-      for (int i = 0; i < 3; ++i) vb[i] = 0.f;
-#pragma unroll
-      for (int i = 0; i < 9; ++i) Ab[i] = 0.f;
-#pragma unroll
-      for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int b = 0; b < 3; ++b)
-#pragma unroll
-          for (int c = 0; c < 3; ++c) {
-            if (!node_ok(sn, a, b, c, k.N)) continue;
-            const float wt = weight(sn, a, b, c);
-            float gw[3], dp[3];
-            weight_grad(sn, a, b, c, gw);
-            node_offset(sn, a, b, c, x, k, dp);
-            const float4 g = gm[node_index(sn, a, b, c, k.N)];
-            const float pb[3] = {g.x, g.y, g.z};
-            float val = g.w * d.mass;  // pb . (m v + A dp) + mb m
-#pragma unroll
-            for (int r = 0; r < 3; ++r) {
-              vb[r] += d.mass * wt * pb[r];
-              val += pb[r] * (d.mass * v[r] + (A[3 * r] * dp[0] + A[3 * r + 1] * dp[1] + A[3 * r + 2] * dp[2]));
-#pragma unroll
-              for (int q = 0; q < 3; ++q) Ab[3 * r + q] += wt * pb[r] * dp[q];
-            }
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-              const float atp = A[q] * pb[0] + A[3 + q] * pb[1] + A[6 + q] * pb[2];  // (A^T pb)_q
-              xb[q] += gw[q] * val - wt * atp;
-            }
-          }
-      // stress adjoint tb = sc Ab; mu and lambda adjoints
-      float tb[9];
-#pragma unroll
-      for (int i = 0; i < 9; ++i) tb[i] = sc * Ab[i];
-      const float J = det3(F);
+      for (int r = 0; r < 3; ++r) q0[r] = d.mass * v[r];
+      // per node, pb . (m v + A dp) + mb m is what its weight multiplies
+      plane_sums<true, true, false>(gm, sn, plane, k.N, q0, A, d.mass, nullptr, s);
+      put_plane<4>(part_p, plane, lane, s);
+    } else {
+      float U[9], sv[3], V[9];
+      svd3_robust(F, U, sv, V);
+      mul_abt(U, V, R);
+    }
+    __syncthreads();
+    sum_planes<4>(part_p, lane, s);
+    if (inside && plane == kPlanes) {
+      const float* Ab = s + 3;
       float FmR[9], FmRFt[9];
 #pragma unroll
       for (int i = 0; i < 9; ++i) FmR[i] = F[i] - R[i];
       mul_abt(FmR, F, FmRFt);
       float dmu = 0.f;
 #pragma unroll
-      for (int i = 0; i < 9; ++i) dmu += FmRFt[i] * tb[i];
-      const float trt = tb[0] + tb[4] + tb[8];
+      for (int i = 0; i < 9; ++i) dmu += FmRFt[i] * (sc * Ab[i]);
+      const float J = det3(F);
       adj_mu[p] += 2.0f * dmu;
-      adj_lam[p] += ((J - 1.0f) * J) * trt;
+      adj_lam[p] += ((J - 1.0f) * J) * (sc * Ab[0] + sc * Ab[4] + sc * Ab[8]);
+    } else if (inside) {
+      const float *pb = s, *Ab = s + 3;  // sum w pb, sum w pb dp^T
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        vb[q] = d.mass * pb[q];
+        xb[q] += s[12 + q] - (A[q] * pb[0] + A[3 + q] * pb[1] + A[6 + q] * pb[2]);
+      }
+      // stress adjoint tb = sc Ab
+      float tb[9];
+#pragma unroll
+      for (int i = 0; i < 9; ++i) tb[i] = sc * Ab[i];
+      const float J = det3(F);
+      float FmR[9];
+#pragma unroll
+      for (int i = 0; i < 9; ++i) FmR[i] = F[i] - R[i];
+      const float trt = tb[0] + tb[4] + tb[8];
       // with R held: d/dF of 2 mu (F - R) F^T contracted with tb = 2 mu (tb F + tb^T (F - R))
       float tbF[9], tbtFmR[9];
       mul_ab(tb, F, tbF);
@@ -460,36 +819,48 @@ __global__ void __launch_bounds__(kWave)
           tbtFmR[3 * r + c] = tb[r] * FmR[c] + tb[3 + r] * FmR[3 + c] + tb[6 + r] * FmR[6 + c];
 #pragma unroll
       for (int i = 0; i < 9; ++i) Fb[i] += 2.0f * mup * (tbF[i] + tbtFmR[i]);
-      // through R: Rbar = -2 mu tb F, M = R^T Rbar
+      // through R: Rbar = -2 mu tb F, M = R^T Rbar, Sk = skew(M)
       float M[9];
 #pragma unroll
       for (int r = 0; r < 3; ++r)
 #pragma unroll
         for (int c = 0; c < 3; ++c)
           M[3 * r + c] = -2.0f * mup * (R[r] * tbF[c] + R[3 + r] * tbF[3 + c] + R[6 + r] * tbF[6 + c]);
-      float Sk[9], T1[9], Mt[9];
+      const float ax[3] = {0.5f * (M[7] - M[5]), 0.5f * (M[2] - M[6]), 0.5f * (M[3] - M[1])};
+      float FbR[9];
+      if (by_svd) {
+        const float Sk[9] = {0.f, -ax[2], ax[1], ax[2], 0.f, -ax[0], -ax[1], ax[0], 0.f};
+        float f[9], o[9];
 #pragma unroll
-      for (int r = 0; r < 3; ++r)
+        for (int i = 0; i < 9; ++i) f[i] = F[i];
+        svd_rotation_adjoint(f, Sk, o);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) Sk[3 * r + c] = 0.5f * (M[3 * r + c] - M[3 * c + r]);
-      mul_ab(Sk, V, T1);  // skew(M) V
+        for (int i = 0; i < 9; ++i) FbR[i] = o[i];
+      } else {
+        // Sk = [ax]x: the skew X with S X + X S = Sk, S = R^T F, is [y]x with
+        // (tr S - S) y = ax (its eigenvalues are the s_i + s_j, above 1/4 here)
+        float S[9];
 #pragma unroll
-      for (int r = 0; r < 3; ++r)
+        for (int r = 0; r < 3; ++r)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) Mt[3 * r + c] = V[r] * T1[c] + V[3 + r] * T1[3 + c] + V[6 + r] * T1[6 + c];
-      float Nm[9];
+          for (int c = 0; c < 3; ++c) S[3 * r + c] = R[r] * F[c] + R[3 + r] * F[3 + c] + R[6 + r] * F[6 + c];
+        const float k00 = S[4] + S[8], k11 = S[0] + S[8], k22 = S[0] + S[4];
+        const float k01 = -0.5f * (S[1] + S[3]), k02 = -0.5f * (S[2] + S[6]), k12 = -0.5f * (S[5] + S[7]);
+        const float c00 = k11 * k22 - k12 * k12, c01 = k02 * k12 - k01 * k22, c02 = k01 * k12 - k02 * k11;
+        const float c11 = k00 * k22 - k02 * k02, c12 = k01 * k02 - k00 * k12, c22 = k00 * k11 - k01 * k01;
+        const float h = 2.0f / (k00 * c00 + k01 * c01 + k02 * c02);
+        const float y0 = h * (c00 * ax[0] + c01 * ax[1] + c02 * ax[2]);
+        const float y1 = h * (c01 * ax[0] + c11 * ax[1] + c12 * ax[2]);
+        const float y2 = h * (c02 * ax[0] + c12 * ax[1] + c22 * ax[2]);
 #pragma unroll
-      for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          const float den = s[r] + s[c];
-          Nm[3 * r + c] = (r == c || den == 0.0f) ? 0.0f : Mt[3 * r + c] / den;
+        for (int r = 0; r < 3; ++r) {  // 2 R [y]x
+          FbR[3 * r] = R[3 * r + 1] * y2 - R[3 * r + 2] * y1;
+          FbR[3 * r + 1] = R[3 * r + 2] * y0 - R[3 * r] * y2;
+          FbR[3 * r + 2] = R[3 * r] * y1 - R[3 * r + 1] * y0;
         }
-      float UN[9], UNVt[9];
-      mul_ab(U, Nm, UN);
-      mul_abt(UN, V, UNVt);
+      }
 #pragma unroll
-      for (int i = 0; i < 9; ++i) Fb[i] += 2.0f * UNVt[i];
+      for (int i = 0; i < 9; ++i) Fb[i] += FbR[i];
       // volumetric: lambda (2J - 1) tr(tb) dJ/dF, dJ/dF = cof(F)
       const float cv = lamp * (2.0f * J - 1.0f) * trt;
       const float cof[9] = {F[4] * F[8] - F[5] * F[7], F[5] * F[6] - F[3] * F[8], F[3] * F[7] - F[4] * F[6],
@@ -499,35 +870,50 @@ __global__ void __launch_bounds__(kWave)
       for (int i = 0; i < 9; ++i) Fb[i] += cv * cof[i];
 #pragma unroll
       for (int i = 0; i < 9; ++i) Cb[i] = d.mass * Ab[i];
+    } else if (valid) {  // the partial already holds the identity map
+      load_planes<3>(adj_src, n, p, DV, vb);
+      load_planes<9>(adj_src, n, p, DC, Cb);
     }
   }
   // (xb, vb, Cb, Fb) is the adjoint of X_s
   if (!G2PA) {
-    if (valid) store_state(adj_dst, n, p, xb, vb, Cb, Fb);
+    // (adj_dst may be adj_src: no wavefront stores before all have read)
+    __syncthreads();
+    if (valid) store_state(adj_dst, n, p, plane, xb, vb, Cb, Fb);
     return;
   }
   // G2P of substep s-1: X_s = G2P(X_{s-1}); the adjoint of X_s flows back
-  // to x and F of X_{s-1} and to the grid velocities of substep s-1
-  int key = -1;
-  Stencil sn;
-  sn.base[0] = sn.base[1] = sn.base[2] = 0;
-  if (valid) {
-    float x[3], F[9];
-    load_xF(st_prev, n, p, x, F);
-    sn = make_stencil(x, k);
-    if (sn.outside) {
-      store_state(adj_dst, n, p, xb, vb, Cb, Fb);  // the identity map
-    } else {
-      float vn[3], Cn[9];
-      g2p_affine(sn, x, vel_prev, k, vn, Cn);
-      // x' = x + dt v', F' = (I + dt C') F: adjoints of v' and C' through them
-      float vbt[3], Cbt[9], FbFt[9];
+  // to x and F of X_{s-1} and to the grid velocities of substep s-1:
+  // x' = x + dt v', F' = (I + dt C') F, adjoints of v' and C' through them
+  const Stencil sn = make_stencil(xp, k);
+  const bool inside = valid && !sn.outside;
+  float vbt[3], D[9], FbFt[9];  // D: Dinv times the adjoint of C'
 #pragma unroll
-      for (int a = 0; a < 3; ++a) vbt[a] = vb[a] + k.dt * xb[a];
-      mul_abt(Fb, F, FbFt);
+  for (int a = 0; a < 3; ++a) vbt[a] = vb[a] + k.dt * xb[a];
+  mul_abt(Fb, Fp, FbFt);
 #pragma unroll
-      for (int i = 0; i < 9; ++i) Cbt[i] = Cb[i] + k.dt * FbFt[i];
-      float xo[3] = {xb[0], xb[1], xb[2]}, Fo[9];
+  for (int i = 0; i < 9; ++i) D[i] = k.dinv * (Cb[i] + k.dt * FbFt[i]);
+  // per node, g . (vbt + D dp) is what its weight multiplies, and w (vbt + D dp)
+  // the adjoint of its velocity
+  float s[16];
+  if (plane < kPlanes) {
+    float4 row[9];
+    plane_sums<true, false, true>(vel_prev, sn, plane, k.N, vbt, D, 0.f, row, s);
+    put_plane<4>(part_g, plane, lane, s);
+    scatter_runs<3>(sh, row, inside, sn, plane, k.N);
+  } else {
+    scatter_cells(sh, inside, sn, k.N);
+  }
+  __syncthreads();  // (also: all have read adj_src before any stores)
+  sum_planes<4>(part_g, lane, s);
+  if (inside) {
+    if (plane == 0) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        xb[q] += s[12 + q] - (D[q] * s[0] + D[3 + q] * s[1] + D[6 + q] * s[2]);
+      store_planes<3>(adj_dst, n, p, DX, xb);
+    } else if (plane == 1) {
+      float Fo[9];
 #pragma unroll
       for (int r = 0; r < 3; ++r)
 #pragma unroll
@@ -535,49 +921,16 @@ __global__ void __launch_bounds__(kWave)
           // ((I + dt C')^T Fb')_rc
           float acc = 0.f;
 #pragma unroll
-          for (int q = 0; q < 3; ++q) acc += (((q == r) ? 1.0f : 0.0f) + k.dt * Cn[3 * q + r]) * Fb[3 * q + c];
+          for (int q = 0; q < 3; ++q)
+            acc += (((q == r) ? 1.0f : 0.0f) + (k.dt * k.dinv) * s[3 + 3 * q + r]) * Fb[3 * q + c];
           Fo[3 * r + c] = acc;
         }
-      float* row = table + lane * kAdjStride;
-#pragma unroll
-      for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int b = 0; b < 3; ++b)
-#pragma unroll
-          for (int c = 0; c < 3; ++c) {
-            const int o = 3 * (9 * a + 3 * b + c);
-            if (!node_ok(sn, a, b, c, k.N)) {
-              row[o] = row[o + 1] = row[o + 2] = 0.0f;
-              continue;
-            }
-            const float wt = weight(sn, a, b, c);
-            float gw[3], dp[3];
-            weight_grad(sn, a, b, c, gw);
-            node_offset(sn, a, b, c, x, k, dp);
-            const float4 gv4 = vel_prev[node_index(sn, a, b, c, k.N)];
-            const float gv[3] = {gv4.x, gv4.y, gv4.z};
-            float Cdp[3];
-#pragma unroll
-            for (int r = 0; r < 3; ++r) Cdp[r] = Cbt[3 * r] * dp[0] + Cbt[3 * r + 1] * dp[1] + Cbt[3 * r + 2] * dp[2];
-            const float s1 = gv[0] * vbt[0] + gv[1] * vbt[1] + gv[2] * vbt[2];
-            const float s2 = gv[0] * Cdp[0] + gv[1] * Cdp[1] + gv[2] * Cdp[2];
-            const float coef = s1 + k.dinv * s2;
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-              const float ctg = Cbt[q] * gv[0] + Cbt[3 + q] * gv[1] + Cbt[6 + q] * gv[2];  // (C'^T g)_q
-              xo[q] += gw[q] * coef - (k.dinv * wt) * ctg;
-            }
-#pragma unroll
-            for (int r = 0; r < 3; ++r) row[o + r] = wt * (vbt[r] + k.dinv * Cdp[r]);
-          }
-#pragma unroll
-      for (int a = 0; a < 3; ++a) adj_dst[(DX + a) * n + p] = xo[a];
-#pragma unroll
-      for (int i = 0; i < 9; ++i) adj_dst[(DF + i) * n + p] = Fo[i];
-      key = cell_key(sn, k.N);
+      store_planes<9>(adj_dst, n, p, DF, Fo);
     }
+  } else if (valid) {
+    store_state(adj_dst, n, p, plane, xb, vb, Cb, Fb);  // the identity map
   }
-  run_scatter<kAdjVals, kAdjStride, 3>(table, key, sn.base, k.N, gv_out);
+  scatter_nodes<3>(sh, plane, k.N, gv_out);
 }
 
 // adjoint of the updated velocity (gadj.xyz) -> adjoints of the P2G momentum
@@ -693,7 +1046,7 @@ hipError_t diff_forward_steps(const StepConsts& k, float mass, float volume, int
   const unsigned gp = particle_blocks(n), gn = node_blocks(k);
   hipLaunchKernelGGL(k_zero4, dim3(gn), dim3(256), 0, s, grid, nodes_of(k));
   if (n > 0)
-    hipLaunchKernelGGL((k_diff_step<false, true>), dim3(gp), dim3(kWave), 0, s, st0, (float*)nullptr,
+    hipLaunchKernelGGL((k_diff_step<false, true>), dim3(gp), dim3(kThreads), 0, s, st0, (float*)nullptr,
                        (const float4*)nullptr, mu, lam, d, (float*)grid);
   for (int32_t j = 0; j < steps; ++j) {
     float* tape = tapes + (size_t)j * (size_t)tape_stride;
@@ -702,10 +1055,10 @@ hipError_t diff_forward_steps(const StepConsts& k, float mass, float volume, int
     const float* in = j == 0 ? st0 : states + (size_t)(j - 1) * (size_t)state_stride;
     float* out = states + (size_t)j * (size_t)state_stride;
     if (j + 1 < steps)
-      hipLaunchKernelGGL((k_diff_step<true, true>), dim3(gp), dim3(kWave), 0, s, in, out,
+      hipLaunchKernelGGL((k_diff_step<true, true>), dim3(gp), dim3(kThreads), 0, s, in, out,
                          (const float4*)tape_v(tape), mu, lam, d, (float*)grid);
     else
-      hipLaunchKernelGGL((k_diff_step<true, false>), dim3(gp), dim3(kWave), 0, s, in, out,
+      hipLaunchKernelGGL((k_diff_step<true, false>), dim3(gp), dim3(kThreads), 0, s, in, out,
                          (const float4*)tape_v(tape), mu, lam, d, (float*)nullptr);
   }
   return hipGetLastError();
@@ -732,7 +1085,7 @@ hipError_t diff_backward_steps(const StepConsts& k, float mass, float volume, in
   hipLaunchKernelGGL(k_zero4, dim3(gn), dim3(256), 0, s, ga, nodes);
   // the G2P adjoint of the last substep, from the caller's adjoint
   if (n > 0)
-    hipLaunchKernelGGL((k_adj_step<false, true>), dim3(gp), dim3(kWave), 0, s, (const float*)nullptr,
+    hipLaunchKernelGGL((k_adj_step<false, true>), dim3(gp), dim3(kThreads), 0, s, (const float*)nullptr,
                        (const float*)nullptr, (const float*)nullptr, (const float4*)nullptr, adj_out,
                        state(steps - 1), tape_v(tape(steps - 1)), work, (float*)nullptr, (float*)nullptr,
                        (float*)ga, d);
@@ -741,14 +1094,14 @@ hipError_t diff_backward_steps(const StepConsts& k, float mass, float volume, in
                        tape_v(tape(j)), tape_w(tape(j), k), k);
     if (n == 0) continue;
     if (j > 0) {
-      hipLaunchKernelGGL((k_adj_step<true, true>), dim3(gp), dim3(kWave), 0, s, state(j), mu, lam,
+      hipLaunchKernelGGL((k_adj_step<true, true>), dim3(gp), dim3(kThreads), 0, s, state(j), mu, lam,
                          (const float4*)ga, (const float*)work, state(j - 1), tape_v(tape(j - 1)), work, adj_mu,
                          adj_lam, (float*)gb, d);
       float4* t = ga;
       ga = gb;
       gb = t;
     } else {
-      hipLaunchKernelGGL((k_adj_step<true, false>), dim3(gp), dim3(kWave), 0, s, state(0), mu, lam,
+      hipLaunchKernelGGL((k_adj_step<true, false>), dim3(gp), dim3(kThreads), 0, s, state(0), mu, lam,
                          (const float4*)ga, (const float*)work, (const float*)nullptr, (const float4*)nullptr,
                          adj_in, adj_mu, adj_lam, (float*)nullptr, d);
     }

@@ -1,0 +1,101 @@
+"""One differentiable substep and its adjoint, against float64 autograd of the
+same step (oracle/diff_torch.py), where the kernels take another way:
+
+  * the scatter: particles whose nodes lie in a box that a workgroup sums node
+    by node, and particles in no order, which go run by run; ends of
+    wavefronts and workgroups; stencils clipped at the faces, particles
+    outside the grid
+  * the rotation: Newton's iteration, and the SVD for particles stretched or
+    crushed past 8 or 1/8 or turned inside out
+
+Tolerances are those of the other tests of the substep: 1e-4 of a field's norm
+forward, 1e-3 for the adjoints."""
+import numpy as np
+import pytest
+
+from mpm_amd import COMPAT_FIXED, Params
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+N = 16
+
+
+def rotations(rng, n):
+    q = np.linalg.qr(rng.standard_normal((n, 3, 3)))[0]
+    q[:, :, 0] *= np.linalg.det(q)[:, None]
+    return q
+
+
+def deformations(kind, rng, n):
+    if kind == "small":
+        return np.eye(3) + 0.1 * rng.uniform(-1, 1, (n, 3, 3))
+    s = np.array([1.4, 1.0, 0.6]) * rng.uniform(0.95, 1.05, (n, 3))
+    if kind == "stretched":  # some within the iteration's range, some past it
+        s *= np.exp(rng.uniform(-np.log(20.0), np.log(20.0), (n, 1)))
+    if kind == "mirrored":
+        s[:, 2] *= -1.0
+    return np.einsum("nij,nj,nkj->nik", rotations(rng, n), s, rotations(rng, n))
+
+
+def svd_rotation(F):
+    """U V^T with U and V rotations: a mirrored F has its smallest singular
+    value negative."""
+    U, _, Vh = torch.linalg.svd(F)
+    sign = torch.sign(torch.linalg.det(U) * torch.linalg.det(Vh)).detach()
+    flip = torch.stack([torch.ones_like(sign), torch.ones_like(sign), sign], 1)
+    return (U * flip[:, None, :]) @ Vh
+
+
+CASES = [("cube", 1, "small"), ("cube", 63, "small"), ("cube", 64, "small"), ("cube", 65, "small"),
+         ("cube", 200, "stretched"), ("cube", 200, "mirrored"), ("one cell", 130, "small"),
+         ("spread", 200, "small"), ("spread", 129, "mirrored"), ("faces", 300, "small")]
+
+
+@pytest.mark.parametrize("where,n,kind", CASES)
+def test_substep_and_adjoint(gpu_lib, monkeypatch, where, n, kind):
+    from mpm_amd.diff import DiffStepper, cell_order, pack_state
+    from oracle import diff_torch
+    monkeypatch.setattr(diff_torch, "polar_rotation", svd_rotation)
+    rng = np.random.default_rng(n)
+    lo, hi = {"cube": (0.4, 0.6), "one cell": (0.44, 0.45), "spread": (0.15, 0.85), "faces": (-0.3, 1.3)}[where]
+    x = rng.uniform(lo, hi, (n, 3)).astype(np.float32)
+    v = rng.uniform(-1, 1, (n, 3)).astype(np.float32)
+    C = rng.uniform(-5, 5, (n, 3, 3)).astype(np.float32)
+    F = deformations(kind, rng, n).astype(np.float32)
+    mu = rng.uniform(0.5, 2.0, n).astype(np.float32) * 1e3
+    lam = rng.uniform(0.5, 2.0, n).astype(np.float32) * 1e3
+    params = Params(dt=1e-4, N=N, gravity=-9.8, compat=COMPAT_FIXED)
+    mass, volume = 1e-3, 1e-6
+    dev = torch.device("cuda")
+    st = pack_state(*(torch.from_numpy(a).to(dev) for a in (x, v, C, F)))
+    mu_t, lam_t = torch.from_numpy(mu).to(dev), torch.from_numpy(lam).to(dev)
+    if where in ("cube", "one cell"):
+        perm = cell_order(st[0:3], N)
+        st, mu_t, lam_t = st[:, perm].contiguous(), mu_t[perm].contiguous(), lam_t[perm].contiguous()
+    s = DiffStepper(params, mass, volume, n)
+    out, adj_in, tape = torch.empty_like(st), torch.empty_like(st), s.new_tape()
+    adj_out = torch.from_numpy(rng.standard_normal((24, n)).astype(np.float32)).to(dev)
+    adj_mu, adj_lam = torch.zeros_like(mu_t), torch.zeros_like(lam_t)
+    s.forward(st, out, mu_t, lam_t, tape)
+    s.backward(st, mu_t, lam_t, tape, adj_out, adj_in, adj_mu, adj_lam)
+    torch.cuda.synchronize()
+
+    st64 = st.cpu().double().requires_grad_(True)
+    mu64, lam64 = mu_t.cpu().double().requires_grad_(True), lam_t.cpu().double().requires_grad_(True)
+    fields = (st64[0:3].T, st64[3:6].T, st64[6:15].T.reshape(n, 3, 3), st64[15:24].T.reshape(n, 3, 3))
+    got = diff_torch.substep(*fields, mu64, lam64, mass, volume, diff_torch.Consts(params))
+    ref = torch.cat([got[0].T, got[1].T, got[2].reshape(n, 9).T, got[3].reshape(n, 9).T])
+    grads = torch.autograd.grad((ref * adj_out.cpu().double()).sum(), [st64, mu64, lam64])
+
+    def off(a, b):
+        return float((a.cpu().double() - b.detach()).norm() / b.detach().norm().clamp(min=1e-30))
+
+    planes = {"x": slice(0, 3), "v": slice(3, 6), "C": slice(6, 15), "F": slice(15, 24)}
+    for k, p in planes.items():
+        assert off(out[p], ref[p]) < 1e-4, (k, off(out[p], ref[p]))
+    for k, p in planes.items():
+        assert off(adj_in[p], grads[0][p]) < 1e-3, (k, off(adj_in[p], grads[0][p]))
+    assert off(adj_mu, grads[1]) < 1e-3, off(adj_mu, grads[1])
+    assert off(adj_lam, grads[2]) < 1e-3, off(adj_lam, grads[2])
