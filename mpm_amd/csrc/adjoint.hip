@@ -12,17 +12,18 @@
 //
 // Kernels, 64 particles and four wavefronts per workgroup (a particle is lane i
 // of each):
-//   k_diff_step<G2P, P2G>   G2P of substep n (gather of the tape velocities,
-//                           F and x update) fused with the P2G of substep n+1
-//                           (stress through the polar rotation of F, scatter)
-//   k_diff_grid             grid update into the tape; clears the grid
+//   k_diff_step<G2P, P2G>   grid update and G2P of substep n (gather of its
+//                           sums, F and x update), fused with the P2G of
+//                           substep n+1 (stress through the polar rotation of
+//                           F, scatter); further workgroups write the grid
+//                           update into the tape
 //   k_adj_step<P2G', G2P'>  the adjoint of the P2G of substep s (gather of the
 //                           momentum and mass adjoints, stress adjoint, mu and
 //                           lambda adjoints) fused with the adjoint of the G2P
 //                           of substep s-1 (scatter of the grid velocity
 //                           adjoint)
 //   k_adj_grid              grid update backward: momentum and mass adjoints
-// so a substep is two launches forward and two backward, and a run of
+// so a substep is one launch forward and two backward, and a run of
 // substeps is enqueued from one host call (diff_forward_steps /
 // diff_backward_steps).
 //
@@ -34,9 +35,10 @@
 // them (storing the state, the cells of the scatter, the SVD of mu's adjoint).
 // A wavefront has its SIMD nearly to itself and runs its code once: short code
 // without branches, in which an LDS or memory round trip is waited for once, is
-// what counts. k_diff_step and k_adj_step took 25 and 38 us for 32,768
-// particles with one wavefront per 64 particles, now 10.2 and 12.6 (2,197
-// particles: 19 and 29, now 7.8 and 9.7).
+// what counts. k_diff_step and k_adj_step took 26 and 38 us for 32,768
+// particles with one wavefront per 64 particles, 10.2 and 12.6 with four
+// (2,197 particles: 19 and 29, then 7.8 and 9.7); k_diff_step takes 11.2 and
+// 8.3 with the grid update, which was a launch of 3 to 5 us.
 //
 // The stress adjoint differentiates the polar rotation R of F = R S: with
 // Rbar the adjoint of R and K = skew(R^T Rbar), Fbar += 2 R X for the skew X
@@ -65,6 +67,7 @@ constexpr int kNowhere = 1 << 20;    // a cell that no node is next to
 struct DiffK {
   StepConsts k;
   float mass, volume;
+  int wall_lo, wall_hi;  // a node index below wall_lo or from wall_hi on is a wall's
   int64_t n;
 };
 
@@ -244,24 +247,75 @@ __device__ __forceinline__ void q_start(const float q0[3], const float M[9], flo
   for (int r = 0; r < 3; ++r) qa[r] = __builtin_fmaf(M[3 * r], dpa, q0[r]);
 }
 
+// The velocity of a node from its momentum and mass (w > 0) before the walls:
+// the quotients, and gravity on y (mpm.cu:76-91). The quotients are c / w to the
+// last bit but in rare cases (q + (c - q w) / w with the reciprocal of a Newton
+// step: Markstein, 1990): with the divisions of the language, each with a
+// serial chain of its own, the 27 of a gather took 2.1 us, these 0.95. The scale
+// keeps a vanishing or a huge mass's reciprocal in range.
+__device__ __forceinline__ void free_velocity(const float4& c, const StepConsts& k, float u[3]) {
+  const float scale = c.w < 0x1p-96f ? 0x1p64f : c.w > 0x1p96f ? 0x1p-64f : 1.0f;
+  const float w = c.w * scale, p[3] = {c.x * scale, c.y * scale, c.z * scale};
+  float r = __builtin_amdgcn_rcpf(w);
+  r = w < __builtin_inff() ? __builtin_fmaf(__builtin_fmaf(-w, r, 1.0f), r, r) : r;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const float q = p[a] * r;
+    u[a] = fabsf(q) < __builtin_inff() ? __builtin_fmaf(__builtin_fmaf(-w, q, p[a]), r, q) : q;
+  }
+  u[1] = __builtin_fmaf(k.dt, k.gravity, u[1]);
+}
+
+// the walls of a node (mpm.cu:92-105): sticky on five sides, a floor
+struct NodeWalls {
+  bool sticky, floor_;
+};
+__device__ __forceinline__ NodeWalls node_walls(int i, int j, int k, const DiffK& d) {
+  NodeWalls w;
+  w.sticky = i < d.wall_lo || i >= d.wall_hi || j >= d.wall_hi || k < d.wall_lo || k >= d.wall_hi;
+  w.floor_ = j < d.wall_lo;
+  return w;
+}
+__device__ __forceinline__ void apply_walls(const NodeWalls& w, float u[3]) {
+#pragma unroll
+  for (int a = 0; a < 3; ++a) u[a] = w.sticky ? 0.0f : u[a];
+  u[1] = w.floor_ ? fmaxf(0.0f, u[1]) : u[1];
+}
+
+__device__ __forceinline__ float4 node_velocity(const float4& sum, int i, int j, int k, const DiffK& d) {
+  float u[3];
+  free_velocity(sum, d.k, u);
+  apply_walls(node_walls(i, j, k, d), u);
+  const bool has = sum.w > 0.0f;
+  return make_float4(has ? u[0] : 0.0f, has ? u[1] : 0.0f, has ? u[2] : 0.0f, 0.0f);
+}
+
 // Sums over the plane of the 4-vectors g = grid[node]:
 //   s[0..2]    sum w g              s[3 + 3 r + q]  sum w g_r dp_q
 // and with GRAD, val = g . (q0 + M dp) + m g.w (m = 0 without MASS),
 //   s[12 + q]  sum (dw/dx_q) val
 // With ROWS the plane's rows w (q0 + M dp) go to `row`.
-template <bool GRAD, bool MASS, bool ROWS>
-__device__ __forceinline__ void plane_sums(const float4* __restrict__ grid, const Stencil& sn, int plane, int N,
-                                           const float q0[3], const float M[9], float m, float4* row,
+// With UPDATE grid holds the momentum and mass sums, updated to velocities here.
+template <bool UPDATE, bool GRAD, bool MASS, bool ROWS>
+__device__ __forceinline__ void plane_sums(const float4* __restrict__ grid, const Stencil& sn, int plane,
+                                           const DiffK& d, const float q0[3], const float M[9], float m, float4* row,
                                            float s[16]) {
   const Axis &ay = sn.ax[1], &az = sn.ax[2];
   const float wa = of_plane(sn.ax[0].w, plane), dpa = of_plane(sn.ax[0].dp, plane);
   const int na = of_plane(sn.ax[0].node, plane);
+  const StepConsts& k = d.k;
   float4 g[9];
 #pragma unroll
   for (int b = 0; b < 3; ++b)
 #pragma unroll
     for (int c = 0; c < 3; ++c)
-      g[3 * b + c] = grid[((size_t)na * N + (size_t)ay.node[b]) * N + (size_t)az.node[c]];
+      g[3 * b + c] = grid[((size_t)na * k.N + (size_t)ay.node[b]) * k.N + (size_t)az.node[c]];
+  if (UPDATE) {
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) g[3 * b + c] = node_velocity(g[3 * b + c], na, ay.node[b], az.node[c], d);
+  }
   float qa[3];
   if (GRAD) q_start(q0, M, dpa, qa);
   float S0[3] = {0.f, 0.f, 0.f}, S1[3] = {0.f, 0.f, 0.f}, S2[3] = {0.f, 0.f, 0.f};
@@ -547,21 +601,63 @@ __device__ __forceinline__ void scatter_nodes(ScatterShared& sh, int wave, int N
 }
 
 // ---------------------------------------------------------------- forward
-// G2P of substep n from `st` with the tape velocities `vel` into `out`
-// (particles outside the grid are copied), fused with the P2G of substep n+1
-// of the new state into `grid`. Without G2P: the P2G of `st`. Without P2G:
-// the G2P only.
+// What the node blocks of a forward launch do, 256 nodes each: the grid update
+// of the substep's momentum and mass `sums` into the tape, tv = (velocity,
+// mass) after the update, tw = (velocity before the walls, wall flags: 1
+// sticky, 2 floor), and the clearing of a later substep's sums. Either may be
+// null.
+struct NodeWork {
+  const float4* sums;
+  float4 *tv, *tw, *clear;
+};
+
+__device__ __forceinline__ void node_block(const NodeWork& w, const DiffK& d, unsigned block) {
+  const int N = d.k.N;
+  const size_t nodes = (size_t)N * N * N;
+  const size_t t = (size_t)block * kThreads + threadIdx.x;
+  if (t >= nodes) return;
+  if (w.clear) w.clear[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (!w.tv) return;
+  const float4 c = w.sums[t];
+  float4 o0 = make_float4(0.f, 0.f, 0.f, c.w), o1 = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (c.w > 0.0f) {
+    // (32-bit: N <= 1024, so a node index is below 2^30)
+    const uint32_t ti = (uint32_t)t, n = (uint32_t)N;
+    const int zi = (int)(ti % n), yi = (int)((ti / n) % n), xi = (int)(ti / (n * n));
+    float u[3];
+    free_velocity(c, d.k, u);
+    const NodeWalls walls = node_walls(xi, yi, zi, d);
+    o1 = make_float4(u[0], u[1], u[2], (float)((walls.sticky ? 1 : 0) | (walls.floor_ ? 2 : 0)));
+    apply_walls(walls, u);
+    o0 = make_float4(u[0], u[1], u[2], c.w);
+  }
+  w.tv[t] = o0;
+  w.tw[t] = o1;
+}
+
+// G2P of substep n from `st` into `out` (particles outside the grid are
+// copied), fused with the P2G of substep n+1 of the new state into `grid`.
+// Without G2P: the P2G of `st`. Without P2G: the G2P only. The first `blocks`
+// workgroups hold the particles, those past them the nodes.
+// The G2P updates the nodes that it gathers by itself, from substep n's sums: 27
+// times as many updates as there are nodes, for 0.95 us of 11.2 (32,768
+// particles), where the grid update as a launch of its own took 3.3 us, a gap
+// and 4 us of the host.
 template <bool G2P, bool P2G>
 __global__ void __launch_bounds__(kThreads)
-    k_diff_step(const float* __restrict__ st, float* __restrict__ out, const float4* __restrict__ vel,
+    k_diff_step(const float* __restrict__ st, float* __restrict__ out, const float4* __restrict__ sums,
                 const float* __restrict__ mu, const float* __restrict__ lam, DiffK d,
-                float* __restrict__ grid) {
+                float* __restrict__ grid, unsigned blocks, NodeWork nodes) {
   __shared__ float4 part[G2P ? kPlanes * 3 * kWave : 1];
   __shared__ ScatterShared sh;  // (unused without P2G, then it takes no LDS)
+  const StepConsts& k = d.k;
+  if (blockIdx.x >= blocks) {
+    node_block(nodes, d, blockIdx.x - blocks);
+    return;
+  }
   const int lane = threadIdx.x & (kWave - 1);
   const int plane = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t p = (int64_t)blockIdx.x * kWave + lane, n = d.n;
-  const StepConsts& k = d.k;
   const bool valid = p < n;
   float x[3] = {0.f, 0.f, 0.f}, v[3] = {0.f, 0.f, 0.f}, C[9], F[9];
 #pragma unroll
@@ -584,7 +680,7 @@ __global__ void __launch_bounds__(kThreads)
   if (G2P) {
     float s[16];
     if (plane < kPlanes) {
-      plane_sums<false, false, false>(vel, sn, plane, k.N, nullptr, nullptr, 0.f, nullptr, s);
+      plane_sums<true, false, false, false>(sums, sn, plane, d, nullptr, nullptr, 0.f, nullptr, s);
       put_plane<3>(part, plane, lane, s);
     }
     __syncthreads();
@@ -647,35 +743,6 @@ __global__ void __launch_bounds__(kThreads)
   }
   __syncthreads();
   scatter_nodes<4>(sh, plane, k.N, grid);
-}
-
-// grid update into the tape: tv = (velocity, mass) after the update, tw =
-// (velocity before the walls, wall flags: 1 sticky, 2 floor); clears the
-// grid for the next scatter
-__global__ void __launch_bounds__(256)
-    k_diff_grid(float4* __restrict__ grid, float4* __restrict__ tv, float4* __restrict__ tw, StepConsts k) {
-  const int N = k.N;
-  const size_t nodes = (size_t)N * N * N;
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nodes) return;
-  const float4 c = grid[t];
-  grid[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-  float4 o0 = make_float4(0.f, 0.f, 0.f, c.w), o1 = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (c.w > 0.0f) {
-    // (32-bit: N <= 1024, so a node index is below 2^30)
-    const uint32_t ti = (uint32_t)t, n = (uint32_t)N;
-    const int zi = (int)(ti % n), yi = (int)((ti / n) % n), xi = (int)(ti / (n * n));
-    o1.x = c.x / c.w;
-    o1.y = __builtin_fmaf(k.dt, k.gravity, c.y / c.w);  // (as grid_node_update rounds it)
-    o1.z = c.z / c.w;
-    const float4 u = grid_node_update(c, xi, yi, zi, k);
-    bool sticky, floor_;
-    wall_flags(xi, yi, zi, k, sticky, floor_);
-    o0 = make_float4(u.x, u.y, u.z, c.w);  // the mass, not the update's w (1)
-    o1.w = (float)((sticky ? 1 : 0) | (floor_ ? 2 : 0));
-  }
-  tv[t] = o0;
-  tw[t] = o1;
 }
 
 // ---------------------------------------------------------------- backward
@@ -772,7 +839,7 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
       for (int r = 0; r < 3; ++r) q0[r] = d.mass * v[r];
       // per node, pb . (m v + A dp) + mb m is what its weight multiplies
-      plane_sums<true, true, false>(gm, sn, plane, k.N, q0, A, d.mass, nullptr, s);
+      plane_sums<false, true, true, false>(gm, sn, plane, d, q0, A, d.mass, nullptr, s);
       put_plane<4>(part_p, plane, lane, s);
     } else {
       float U[9], sv[3], V[9];
@@ -898,7 +965,7 @@ __global__ void __launch_bounds__(kThreads)
   float s[16];
   if (plane < kPlanes) {
     float4 row[9];
-    plane_sums<true, false, true>(vel_prev, sn, plane, k.N, vbt, D, 0.f, row, s);
+    plane_sums<false, true, false, true>(vel_prev, sn, plane, d, vbt, D, 0.f, row, s);
     put_plane<4>(part_g, plane, lane, s);
     scatter_runs<3>(sh, row, inside, sn, plane, k.N);
   } else {
@@ -972,6 +1039,23 @@ DiffK diff_consts(const StepConsts& k, float mass, float volume, int64_t n) {
   d.k = k;
   d.mass = mass;
   d.volume = volume;
+  // wall_flags' comparisons as node indices: i / N grows with i
+  d.wall_lo = k.bcells;
+  d.wall_hi = k.N - k.bcells;
+  if (k.boundary_mode != MPM_BOUNDARY_CELLS) {
+    auto first = [&](auto past) {
+      int lo = 0, hi = k.N;
+      while (lo < hi) {
+        const int mid = (lo + hi) / 2;
+        if (past((float)mid / (float)k.N)) hi = mid;
+        else lo = mid + 1;
+      }
+      return lo;
+    };
+    const float top = 1.0f - k.bfrac;
+    d.wall_lo = first([&](float f) { return !(f < k.bfrac); });
+    d.wall_hi = first([&](float f) { return f > top; });
+  }
   d.n = n;
   return d;
 }
@@ -1038,28 +1122,45 @@ hipError_t diff_forward_noalloc(const StepConsts& k, float mass, float volume, i
 }
 
 
+// A substep's launch reads the sums of its own scatter, adds up the next
+// substep's and clears those of the one after: three grids are in use at a
+// time. With a tape for each substep, the sums of substep j lie in the tape of
+// substep j + 1, which is written after they were read (the last substep's in
+// `grid`); with one tape for all, in `grid` and its two halves in turn, and
+// only the last substep, whose sums are in `grid`, writes it.
 hipError_t diff_forward_steps(const StepConsts& k, float mass, float volume, int64_t n, int32_t steps,
                               const float* st0, float* states, int64_t state_stride, const float* mu,
                               const float* lam, float4* grid, float* tapes, int64_t tape_stride,
                               hipStream_t s) {
   const DiffK d = diff_consts(k, mass, volume, n);
   const unsigned gp = particle_blocks(n), gn = node_blocks(k);
-  hipLaunchKernelGGL(k_zero4, dim3(gn), dim3(256), 0, s, grid, nodes_of(k));
-  if (n > 0)
-    hipLaunchKernelGGL((k_diff_step<false, true>), dim3(gp), dim3(kThreads), 0, s, st0, (float*)nullptr,
-                       (const float4*)nullptr, mu, lam, d, (float*)grid);
+  auto tape = [&](int32_t j) { return tapes + (size_t)j * (size_t)tape_stride; };
+  auto sums = [&](int32_t j) -> float4* {
+    if (j >= steps) return nullptr;
+    const int32_t left = steps - 1 - j;
+    if (tape_stride > 0) return left == 0 ? grid : tape_v(tape(j + 1));
+    return left % 3 == 0 ? grid : left % 3 == 1 ? tape_v(tapes) : tape_w(tapes, k);
+  };
+  if (steps < 1) return hipGetLastError();
+  hipLaunchKernelGGL(k_zero4, dim3(gn), dim3(256), 0, s, sums(0), nodes_of(k));
+  if (n > 0 || steps > 1) {
+    const NodeWork w = {nullptr, nullptr, nullptr, sums(1)};
+    hipLaunchKernelGGL((k_diff_step<false, true>), dim3(gp + (steps > 1 ? gn : 0u)), dim3(kThreads), 0, s, st0,
+                       (float*)nullptr, (const float4*)nullptr, mu, lam, d, (float*)sums(0), gp, w);
+  }
   for (int32_t j = 0; j < steps; ++j) {
-    float* tape = tapes + (size_t)j * (size_t)tape_stride;
-    hipLaunchKernelGGL(k_diff_grid, dim3(gn), dim3(256), 0, s, grid, tape_v(tape), tape_w(tape, k), k);
-    if (n == 0) continue;
     const float* in = j == 0 ? st0 : states + (size_t)(j - 1) * (size_t)state_stride;
     float* out = states + (size_t)j * (size_t)state_stride;
-    if (j + 1 < steps)
-      hipLaunchKernelGGL((k_diff_step<true, true>), dim3(gp), dim3(kThreads), 0, s, in, out,
-                         (const float4*)tape_v(tape), mu, lam, d, (float*)grid);
+    const bool last = j + 1 == steps, taped = last || tape_stride > 0;
+    const NodeWork w = {sums(j), taped ? tape_v(tape(j)) : nullptr, taped ? tape_w(tape(j), k) : nullptr, sums(j + 2)};
+    const unsigned blocks = gp + (w.tv || w.clear ? gn : 0u);
+    if (blocks == 0) continue;
+    if (!last)
+      hipLaunchKernelGGL((k_diff_step<true, true>), dim3(blocks), dim3(kThreads), 0, s, in, out, (const float4*)w.sums,
+                         mu, lam, d, (float*)sums(j + 1), gp, w);
     else
-      hipLaunchKernelGGL((k_diff_step<true, false>), dim3(gp), dim3(kThreads), 0, s, in, out,
-                         (const float4*)tape_v(tape), mu, lam, d, (float*)nullptr);
+      hipLaunchKernelGGL((k_diff_step<true, false>), dim3(blocks), dim3(kThreads), 0, s, in, out, (const float4*)w.sums,
+                         mu, lam, d, (float*)nullptr, gp, w);
   }
   return hipGetLastError();
 }

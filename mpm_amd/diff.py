@@ -8,7 +8,8 @@ checkpointing: the forward keeps the state every `checkpoint_every`
 substeps; the backward recomputes each segment's states and grid tapes from
 its checkpoint (mpm_diff_forward_steps), then runs the segment's adjoints in
 reverse (mpm_diff_backward_steps). Each segment is one call into the
-library, which enqueues all of its kernels (two per substep each way). The
+library, which enqueues all of its kernels (one per substep forward, two
+backward). The
 recompute of segment s - 1 runs on a second stream while segment s's
 adjoints run (two buffers of states and tapes): a cube of a few ten
 thousand particles fills half the SIMDs, and each pass is latency-bound.

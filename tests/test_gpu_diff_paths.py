@@ -99,3 +99,45 @@ def test_substep_and_adjoint(gpu_lib, monkeypatch, where, n, kind):
         assert off(adj_in[p], grads[0][p]) < 1e-3, (k, off(adj_in[p], grads[0][p]))
     assert off(adj_mu, grads[1]) < 1e-3, off(adj_mu, grads[1])
     assert off(adj_lam, grads[2]) < 1e-3, off(adj_lam, grads[2])
+
+
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5])
+def test_runs_of_substeps_with_and_without_tapes(gpu_lib, steps):
+    """A run of substeps keeps the sums of three substeps at a time in the
+    scatter grid and the tapes: the same states and the same last tape one
+    substep at a time, in a run with a tape each and in a run with one tape.
+    The scatters add in any order: 1e-5 of the norm, for at most 5 substeps."""
+    from mpm_amd.diff import DiffStepper, cell_order, pack_state
+    rng = np.random.default_rng(steps)
+    n = 500
+    dev = torch.device("cuda")
+    x = rng.uniform(0.3, 0.7, (n, 3)).astype(np.float32)
+    v = rng.uniform(-1, 1, (n, 3)).astype(np.float32)
+    F = deformations("small", rng, n).astype(np.float32)
+    st = pack_state(*(torch.from_numpy(a).to(dev) for a in (x, v, np.zeros((n, 3, 3), np.float32), F)))
+    st = st[:, cell_order(st[0:3], N)].contiguous()
+    mu, lam = torch.full((n,), 1e3, device=dev), torch.full((n,), 1.5e3, device=dev)
+    s = DiffStepper(Params(dt=1e-4, N=N, gravity=-9.8, compat=COMPAT_FIXED), 1e-3, 1e-6, n)
+    one, tape, cur = [], s.new_tape(), st
+    for _ in range(steps):
+        nxt = torch.empty_like(st)
+        s.forward(cur, nxt, mu, lam, tape)
+        one.append(nxt)
+        cur = nxt
+    got = torch.empty((steps, 24, n), device=dev)
+    tapes = s.new_tapes(steps)
+    s.forward_steps(st, got, mu, lam, tapes)
+    shared = torch.empty_like(got)
+    s.forward_steps(st, shared, mu, lam)
+    torch.cuda.synchronize()
+
+    def off(a, b):
+        return float((a.double() - b.double()).norm() / b.double().norm())
+
+    for j in range(steps):
+        assert off(got[j], one[j]) < 1e-5 and off(shared[j], one[j]) < 1e-5, j
+    nodes = N ** 3
+    a, b = tapes[-1].view(2, nodes, 4), tape.view(2, nodes, 4)
+    heavy = b[0, :, 3] > 1e-6 * b[0, :, 3].max()  # (a vanishing mass's velocity is all rounding)
+    assert off(a[0, heavy], b[0, heavy]) < 1e-4 and off(a[1, heavy], b[1, heavy]) < 1e-4
+    assert torch.equal(a[0, :, 3] > 0, b[0, :, 3] > 0) and torch.equal(a[1, heavy][:, 3], b[1, heavy][:, 3])
