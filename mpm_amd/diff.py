@@ -35,6 +35,7 @@ from __future__ import annotations
 import ctypes as C
 from typing import Tuple
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -166,9 +167,16 @@ class DiffStepper:
 class _Rollout(torch.autograd.Function):
     @staticmethod
     def forward(ctx, stepper: DiffStepper, steps: int, every: int, st0, mu, lam):
-        st0 = st0.detach().contiguous()
-        mu = mu.detach().contiguous()
-        lam = lam.detach().contiguous()
+        # the particles in cell order from here to the results. The gradients
+        # are put back with the inverse permutation: autograd's own backward of
+        # an index sorts it first, which took 0.25 ms of a rollout's 3.9 with
+        # 32,768 particles and 100 substeps.
+        perm = cell_order(st0[0:3], stepper.params.N)
+        inv = torch.empty_like(perm)
+        inv[perm] = torch.arange(perm.numel(), device=perm.device)
+        st0 = st0.index_select(1, perm)
+        mu = mu.index_select(0, perm)
+        lam = lam.index_select(0, perm)
         seg = torch.empty((min(every, steps), PLANES, stepper.n), device=st0.device, dtype=torch.float32)
         cur = st0
         checkpoints = [st0]
@@ -189,14 +197,14 @@ class _Rollout(torch.autograd.Function):
                 checkpoints.append(cur)
         ctx.stepper, ctx.steps, ctx.every = stepper, steps, every
         ctx.checkpoints = checkpoints
-        ctx.save_for_backward(mu, lam)
-        return cur
+        ctx.save_for_backward(mu, lam, perm, inv)
+        return cur.index_select(1, inv)
 
     @staticmethod
     def backward(ctx, g):
         stepper, steps, every = ctx.stepper, ctx.steps, ctx.every
-        mu, lam = ctx.saved_tensors
-        adj = g.detach().to(torch.float32).contiguous().clone()
+        mu, lam, perm, inv = ctx.saved_tensors
+        adj = g.detach().to(torch.float32).index_select(1, perm)
         adj_next = torch.empty_like(adj)
         adj_mu = torch.zeros_like(mu)
         adj_lam = torch.zeros_like(lam)
@@ -244,18 +252,17 @@ class _Rollout(torch.autograd.Function):
         for t in states + tapes:
             t.record_stream(side)
         ctx.checkpoints = None
-        return None, None, None, adj, adj_mu, adj_lam
+        return (None, None, None, adj.index_select(1, inv), adj_mu.index_select(0, inv),
+                adj_lam.index_select(0, inv))
 
 
 def cell_order(x: torch.Tensor, N: int) -> torch.Tensor:
     """Stable order of the particles (positions x: (3, n)) by the base cell
     of their quadratic stencil, int(x / dx - 0.5) per axis."""
-    dx_inv = float(torch.tensor(1.0 / float(torch.tensor(1.0 / N, dtype=torch.float32)),
-                                dtype=torch.float32))
-    b = torch.trunc(x * dx_inv - 0.5).to(torch.int64) + 3
+    dx_inv = float(np.float32(1.0 / float(np.float32(1.0 / N))))
+    b = (x * dx_inv - 0.5).to(torch.int64)  # (the conversion truncates)
     M = N + 3
-    key = (b[0] * M + b[1]) * M + b[2]
-    return torch.argsort(key, stable=True)
+    return torch.argsort(torch.add(torch.add(b[2], b[1], alpha=M), b[0], alpha=M * M), stable=True)
 
 
 def rollout(stepper: DiffStepper, state0: torch.Tensor, mu: torch.Tensor, lam: torch.Tensor,
@@ -266,9 +273,4 @@ def rollout(stepper: DiffStepper, state0: torch.Tensor, mu: torch.Tensor, lam: t
         raise ValueError("steps and checkpoint_every must be >= 1")
     if state0.shape != (PLANES, stepper.n) or mu.shape != (stepper.n,) or lam.shape != (stepper.n,):
         raise ValueError("state0 must be (24, n) and mu, lam (n,)")
-    with torch.no_grad():
-        perm = cell_order(state0[0:3].detach(), stepper.params.N)
-        inv = torch.empty_like(perm)
-        inv[perm] = torch.arange(perm.numel(), device=perm.device)
-    out = _Rollout.apply(stepper, int(steps), int(checkpoint_every), state0[:, perm], mu[perm], lam[perm])
-    return out[:, inv]
+    return _Rollout.apply(stepper, int(steps), int(checkpoint_every), state0, mu, lam)
