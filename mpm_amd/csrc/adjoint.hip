@@ -32,17 +32,20 @@
 // (200 bytes a particle, 6.5 MB) takes 1.3 us at the copy rate. So three
 // wavefronts take an x-plane of the stencil each and run what needs a whole
 // particle (stress, F) side by side, a fourth takes what does not wait for
-// them (storing the state, the cells of the scatter, the SVD of mu's adjoint).
+// them (storing the state, the cells of the scatter, mu's adjoint).
 // A wavefront has its SIMD nearly to itself and runs its code once: short code
 // without branches, in which an LDS or memory round trip is waited for once, is
 // what counts. k_diff_step and k_adj_step took 26 and 38 us for 32,768
-// particles with one wavefront per 64 particles, 10.2 and 12.6 with four
-// (2,197 particles: 19 and 29, then 7.8 and 9.7); k_diff_step takes 11.2 and
-// 8.3 with the grid update, which was a launch of 3 to 5 us.
+// particles with one wavefront per 64 particles, now 12.2 and 13.6, the grid
+// update of 3 to 5 us in the first (2,197 particles: 19 and 29, now 9.6 and
+// 11.4). The SVD's serial chain is 2 us of each. Newton's iteration for the
+// rotation takes 0.6, but the position's adjoint is what is left of momenta
+// that cancel: the last bits by which the rotations differ come out as 1e-3 of
+// its root mean square in sparse cells.
 //
-// The stress adjoint differentiates the polar rotation R of F = R S: with
-// Rbar the adjoint of R and K = skew(R^T Rbar), Fbar += 2 R X for the skew X
-// with S X + X S = K.
+// The stress adjoint differentiates the polar rotation R of F = U S V^T:
+// with Rbar the adjoint of R and M = V^T skew(R^T Rbar) V,
+// Fbar += 2 U N V^T, N_ij = M_ij / (s_i + s_j).
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -152,68 +155,6 @@ __device__ __forceinline__ void store_state(float* st, int64_t n, int64_t p, int
   } else if (plane == 2) {
     store_planes<9>(st, n, p, DF, F);
   }
-}
-
-// ---------------------------------------------------------------- rotation
-// The SVD for the particles polar_rotation leaves: out of line, so that its
-// registers do not count against the kernels'.
-__device__ __noinline__ void svd_rotation(const float* F, float* R) {
-  float U[9], s[3], V[9];
-  svd3_robust(F, U, s, V);
-  mul_abt(U, V, R);
-}
-
-// The polar rotation R of F = R S. Newton's iteration X <- (X + X^-T) / 2
-// (Higham, "Computing the polar decomposition", 1986) from X = F: with
-// singular values in (1/8, 8) and det F > 0 it converges quadratically to the
-// rotation that U V^T of the SVD is, and its 42 operations a step have nothing
-// serial but the determinant's reciprocal. A solid that is deformed by 1 %
-// takes 3 steps, with the stress 0.6 us (1,500 cycles) of a wavefront that has
-// its SIMD to itself, where the Jacobi SVD's chain of 12 rotations, sort and QR
-// is 870 instructions, over 2 us. The other particles (turned inside out,
-// crushed or drawn out, not finite) go through the SVD; returns whether this
-// lane's did. Every lane of the wavefront calls it.
-__device__ __forceinline__ bool polar_rotation(const float F[9], bool live, float R[9]) {
-  float X[9];
-#pragma unroll
-  for (int i = 0; i < 9; ++i) X[i] = F[i];
-  bool bad = false, done = !live;
-  for (int it = 0; it < 8; ++it) {
-    const float cof[9] = {X[4] * X[8] - X[5] * X[7], X[5] * X[6] - X[3] * X[8], X[3] * X[7] - X[4] * X[6],
-                          X[2] * X[7] - X[1] * X[8], X[0] * X[8] - X[2] * X[6], X[1] * X[6] - X[0] * X[7],
-                          X[1] * X[5] - X[2] * X[4], X[2] * X[3] - X[0] * X[5], X[0] * X[4] - X[1] * X[3]};
-    const float det = X[0] * cof[0] + X[1] * cof[1] + X[2] * cof[2];
-    const float h = 0.5f / det;
-    float step = 0.0f, size = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-      const float y = __builtin_fmaf(h, cof[i], 0.5f * X[i]);
-      const float dx = y - X[i];
-      step += dx * dx;
-      size += y * y;
-      X[i] = y;
-    }
-    // after one step a singular value s has become (s + 1/s) / 2: above 4.06
-    // for s past 8 or 1/8
-    if (it == 0) bad = !(det > 0.0f) || !(size < 16.5f);
-    // (the step's length is the error before it, half its square the one after)
-    done |= bad || step < 1e-7f;
-    if (__ballot(!done) == 0ull) break;
-  }
-  bad = live && (bad || !done);
-#pragma unroll
-  for (int i = 0; i < 9; ++i) R[i] = X[i];
-  if (bad) {
-    // (the copies are the arrays whose address the call takes: F and R of the
-    // common path stay in registers)
-    float f[9], r[9];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) f[i] = F[i];
-    svd_rotation(f, r);
-#pragma unroll
-    for (int i = 0; i < 9; ++i) R[i] = r[i];
-  }
-  return bad;
 }
 
 // tau = 2 mu (F - R) F^T + lambda (J - 1) J I, J = det F
@@ -422,8 +363,8 @@ struct ScatterShared {
 //                  workgroup's particles reach, adds up the runs that touch it
 //                  and sends the sum to `grid`
 // 32,768 particles at 25 a cell have 4 runs in a workgroup at the start of a
-// rollout and 19 (of 8 cells) after 100 substeps, and reach 54 and 82 nodes,
-// where an atomic per run and node makes 100 and 520: 100 substeps take 2.86
+// rollout and 19 (of 8 cells) after 100 substeps, and reach 49 and 74 nodes,
+// where an atomic per run and node makes 100 and 520: 100 substeps took 2.86
 // ms with the runs' atomics alone and 1.72 summed by node. Tried besides: a
 // walk over the 64 rows (50 cycles a row unrolled, 200 in a loop: 5 us and
 // more), and LDS atomics into the box, run by run (a wavefront's 64 lanes take
@@ -640,7 +581,7 @@ __device__ __forceinline__ void node_block(const NodeWork& w, const DiffK& d, un
 // Without G2P: the P2G of `st`. Without P2G: the G2P only. The first `blocks`
 // workgroups hold the particles, those past them the nodes.
 // The G2P updates the nodes that it gathers by itself, from substep n's sums: 27
-// times as many updates as there are nodes, for 0.95 us of 11.2 (32,768
+// times as many updates as there are nodes, for 0.95 us of 12.2 (32,768
 // particles), where the grid update as a launch of its own took 3.3 us, a gap
 // and 4 us of the host.
 template <bool G2P, bool P2G>
@@ -717,8 +658,9 @@ __global__ void __launch_bounds__(kThreads)
   if (plane == kPlanes) {
     scatter_cells(sh, inside, sn, k.N);
   } else {
-    float R[9], tau[9], A[9];
-    polar_rotation(F, inside, R);
+    float U[9], sv[3], V[9], R[9], tau[9], A[9];
+    svd3_robust(F, U, sv, V);
+    mul_abt(U, V, R);
     fc_stress(F, R, mup, lamp, tau);
     const float sc = stress_scale(d);
     float q0[3], qa[3];
@@ -746,25 +688,6 @@ __global__ void __launch_bounds__(kThreads)
 }
 
 // ---------------------------------------------------------------- backward
-// The part of the adjoint of F that comes through its rotation: 2 U N V^T,
-// N_ij = (V^T Sk V)_ij / (s_i + s_j), for the particles whose rotation came
-// from the SVD.
-__device__ __noinline__ void svd_rotation_adjoint(const float* F, const float* Sk, float* out) {
-  float U[9], s[3], V[9], T1[9], Nm[9], UN[9];
-  svd3_robust(F, U, s, V);
-  mul_ab(Sk, V, T1);
-#pragma unroll
-  for (int r = 0; r < 3; ++r)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const float mt = V[r] * T1[c] + V[3 + r] * T1[3 + c] + V[6 + r] * T1[6 + c];
-      const float den = s[r] + s[c];
-      Nm[3 * r + c] = (r == c || den == 0.0f) ? 0.0f : 2.0f * mt / den;
-    }
-  mul_ab(U, Nm, UN);
-  mul_abt(UN, V, out);
-}
-
 // The adjoint of the P2G of substep s (P2GA: the momentum and mass adjoints
 // `gm` of that substep, gathered) fused with the adjoint of the G2P of
 // substep s-1 (G2PA: the grid velocity adjoint scattered into `gv_out`).
@@ -776,10 +699,7 @@ __device__ __noinline__ void svd_rotation_adjoint(const float* F, const float* S
 // X_s = st_s (state before substep s), X_{s-1} = st_prev with tape velocities
 // vel_prev. The mu and lambda adjoints are added into adj_mu, adj_lam.
 //
-// The fourth wavefront takes the mu and lambda adjoints off the others:
-// mu's is (F - R) F^T : tb, and F - R of a solid deformed by 1 % turns an
-// error of R into one a hundred times larger, so its R stays the SVD's, whose
-// chain the wavefront runs while the planes gather.
+// The fourth wavefront takes the mu and lambda adjoints off the others.
 template <bool P2GA, bool G2PA>
 __global__ void __launch_bounds__(kThreads)
     k_adj_step(const float* __restrict__ st_s, const float* __restrict__ mu, const float* __restrict__ lam,
@@ -827,12 +747,12 @@ __global__ void __launch_bounds__(kThreads)
     }
     const Stencil sn = make_stencil(x, k);
     const bool inside = valid && !sn.outside;
-    float R[9], tau[9], A[9], q0[3];
-    bool by_svd = false;
+    float U[9], sv[3], V[9], R[9], tau[9], A[9], q0[3];
     const float sc = stress_scale(d);
     float s[16];
+    svd3_robust(F, U, sv, V);
+    mul_abt(U, V, R);
     if (plane < kPlanes) {
-      by_svd = polar_rotation(F, inside, R);
       fc_stress(F, R, mup, lamp, tau);
 #pragma unroll
       for (int i = 0; i < 9; ++i) A[i] = sc * tau[i] + d.mass * C[i];
@@ -841,10 +761,6 @@ __global__ void __launch_bounds__(kThreads)
       // per node, pb . (m v + A dp) + mb m is what its weight multiplies
       plane_sums<false, true, true, false>(gm, sn, plane, d, q0, A, d.mass, nullptr, s);
       put_plane<4>(part_p, plane, lane, s);
-    } else {
-      float U[9], sv[3], V[9];
-      svd3_robust(F, U, sv, V);
-      mul_abt(U, V, R);
     }
     __syncthreads();
     sum_planes<4>(part_p, lane, s);
@@ -886,48 +802,31 @@ __global__ void __launch_bounds__(kThreads)
           tbtFmR[3 * r + c] = tb[r] * FmR[c] + tb[3 + r] * FmR[3 + c] + tb[6 + r] * FmR[6 + c];
 #pragma unroll
       for (int i = 0; i < 9; ++i) Fb[i] += 2.0f * mup * (tbF[i] + tbtFmR[i]);
-      // through R: Rbar = -2 mu tb F, M = R^T Rbar, Sk = skew(M)
+      // through R: Rbar = -2 mu tb F, M = R^T Rbar
       float M[9];
 #pragma unroll
       for (int r = 0; r < 3; ++r)
 #pragma unroll
         for (int c = 0; c < 3; ++c)
           M[3 * r + c] = -2.0f * mup * (R[r] * tbF[c] + R[3 + r] * tbF[3 + c] + R[6 + r] * tbF[6 + c]);
-      const float ax[3] = {0.5f * (M[7] - M[5]), 0.5f * (M[2] - M[6]), 0.5f * (M[3] - M[1])};
-      float FbR[9];
-      if (by_svd) {
-        const float Sk[9] = {0.f, -ax[2], ax[1], ax[2], 0.f, -ax[0], -ax[1], ax[0], 0.f};
-        float f[9], o[9];
+      float Sk[9], T1[9], Nm[9], UN[9], UNVt[9];
 #pragma unroll
-        for (int i = 0; i < 9; ++i) f[i] = F[i];
-        svd_rotation_adjoint(f, Sk, o);
+      for (int r = 0; r < 3; ++r)
 #pragma unroll
-        for (int i = 0; i < 9; ++i) FbR[i] = o[i];
-      } else {
-        // Sk = [ax]x: the skew X with S X + X S = Sk, S = R^T F, is [y]x with
-        // (tr S - S) y = ax (its eigenvalues are the s_i + s_j, above 1/4 here)
-        float S[9];
+        for (int c = 0; c < 3; ++c) Sk[3 * r + c] = 0.5f * (M[3 * r + c] - M[3 * c + r]);
+      mul_ab(Sk, V, T1);  // skew(M) V
 #pragma unroll
-        for (int r = 0; r < 3; ++r)
+      for (int r = 0; r < 3; ++r)
 #pragma unroll
-          for (int c = 0; c < 3; ++c) S[3 * r + c] = R[r] * F[c] + R[3 + r] * F[3 + c] + R[6 + r] * F[6 + c];
-        const float k00 = S[4] + S[8], k11 = S[0] + S[8], k22 = S[0] + S[4];
-        const float k01 = -0.5f * (S[1] + S[3]), k02 = -0.5f * (S[2] + S[6]), k12 = -0.5f * (S[5] + S[7]);
-        const float c00 = k11 * k22 - k12 * k12, c01 = k02 * k12 - k01 * k22, c02 = k01 * k12 - k02 * k11;
-        const float c11 = k00 * k22 - k02 * k02, c12 = k01 * k02 - k00 * k12, c22 = k00 * k11 - k01 * k01;
-        const float h = 2.0f / (k00 * c00 + k01 * c01 + k02 * c02);
-        const float y0 = h * (c00 * ax[0] + c01 * ax[1] + c02 * ax[2]);
-        const float y1 = h * (c01 * ax[0] + c11 * ax[1] + c12 * ax[2]);
-        const float y2 = h * (c02 * ax[0] + c12 * ax[1] + c22 * ax[2]);
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {  // 2 R [y]x
-          FbR[3 * r] = R[3 * r + 1] * y2 - R[3 * r + 2] * y1;
-          FbR[3 * r + 1] = R[3 * r + 2] * y0 - R[3 * r] * y2;
-          FbR[3 * r + 2] = R[3 * r] * y1 - R[3 * r + 1] * y0;
+        for (int c = 0; c < 3; ++c) {
+          const float mt = V[r] * T1[c] + V[3 + r] * T1[3 + c] + V[6 + r] * T1[6 + c];
+          const float den = sv[r] + sv[c];
+          Nm[3 * r + c] = (r == c || den == 0.0f) ? 0.0f : mt / den;
         }
-      }
+      mul_ab(U, Nm, UN);
+      mul_abt(UN, V, UNVt);
 #pragma unroll
-      for (int i = 0; i < 9; ++i) Fb[i] += FbR[i];
+      for (int i = 0; i < 9; ++i) Fb[i] += 2.0f * UNVt[i];
       // volumetric: lambda (2J - 1) tr(tb) dJ/dF, dJ/dF = cof(F)
       const float cv = lamp * (2.0f * J - 1.0f) * trt;
       const float cof[9] = {F[4] * F[8] - F[5] * F[7], F[5] * F[6] - F[3] * F[8], F[3] * F[7] - F[4] * F[6],

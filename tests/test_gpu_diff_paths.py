@@ -5,8 +5,7 @@ same step (oracle/diff_torch.py), where the kernels take another way:
     by node, and particles in no order, which go run by run; ends of
     wavefronts and workgroups; stencils clipped at the faces, particles
     outside the grid
-  * the rotation: Newton's iteration, and the SVD for particles stretched or
-    crushed past 8 or 1/8 or turned inside out
+  * the rotation: particles stretched, crushed or turned inside out
 
 Tolerances are those of the other tests of the substep: 1e-4 of a field's norm
 forward, 1e-3 for the adjoints."""
@@ -32,7 +31,7 @@ def deformations(kind, rng, n):
     if kind == "small":
         return np.eye(3) + 0.1 * rng.uniform(-1, 1, (n, 3, 3))
     s = np.array([1.4, 1.0, 0.6]) * rng.uniform(0.95, 1.05, (n, 3))
-    if kind == "stretched":  # some within the iteration's range, some past it
+    if kind == "stretched":
         s *= np.exp(rng.uniform(-np.log(20.0), np.log(20.0), (n, 1)))
     if kind == "mirrored":
         s[:, 2] *= -1.0
