@@ -411,8 +411,8 @@ bool all_at_cycle_start(const mpm_batch_s* b, int* cycle);
 // With several chains (chain_scenes) chain c > 0 runs on batch stream c - 1,
 // forked from the origin: the chains touch disjoint scenes, and each fills
 // the others' gaps and tails (a launch's last, partly occupied round of
-// workgroups). Either way the chains fork once and join once, so their
-// substeps drift apart and one chain's grid update meets the other's fused
+// workgroups). Either way the substeps' launches fork once and join once, so
+// the chains drift apart and one chain's grid update meets the other's fused
 // pass. Eager substeps are planned first, all their tables copied at once and
 // then launched: with a copy, a fork and a join for every substep, 42 substeps
 // of 24 scenes (5,000 to 120,000 particles) took 9.4 ms, 16 at a time 8.7.
@@ -484,10 +484,17 @@ int run_scenes_fused(mpm_batch_s* b, int32_t n, bool eager, int32_t* ran, size_t
   tw = TableWriter{b, b->h_eager[slot], b->d_eager, b->eager_cap};
   std::vector<std::vector<Chain>> steps;
   int cycle = 0;
+  // Planning may enqueue work of its own on the chains' streams (a scene's F
+  // planes written out): they wait for the origin before it, for the last
+  // call's kernels, and again after the tables' copy.
+  int rc = fork();
   do {
     steps.emplace_back();
-    const int rc = plan(steps.back());
-    if (rc) return rc;
+    if (!rc) rc = plan(steps.back());
+    if (rc) {
+      (void)join();
+      return rc;
+    }
     *ran = (int32_t)steps.size();
   } while (*ran < std::min<int32_t>(n, kEagerSpan) &&
            !(b->use_graph && all_at_cycle_start(b, &cycle) && n - *ran >= cycle));
@@ -496,7 +503,7 @@ int run_scenes_fused(mpm_batch_s* b, int32_t n, bool eager, int32_t* ran, size_t
   if (tw.used)
     BCHK(hipMemcpyAsync(b->d_eager, b->h_eager[slot], tw.used, hipMemcpyHostToDevice, b->origin),
          "hipMemcpyAsync(batch tables)");
-  int rc = fork();
+  rc = fork();
   for (size_t i = 0; i < steps.size() && !rc; ++i) rc = launch(steps[i]);
   const int rj = join();
   if (rc || rj) return rc ? rc : rj;

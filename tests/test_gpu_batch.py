@@ -104,6 +104,37 @@ def test_batch_chains_equal_individual_runs(gpu_lib, chains):
         e.close()
 
 
+@pytest.mark.parametrize("graph", [0, 1])
+def test_batch_after_derive_f_is_switched_off(gpu_lib, graph):
+    """Liquid scenes leave F implicit while derive_f is on; once it is switched
+    off the next advance writes their F planes out first, on the stream of each
+    scene's chain and behind the last call's kernels. Nothing waits for the
+    device in between: the same bits as the scenes alone."""
+    scs = [scenes.small_scene(MATERIAL_WC_LIQUID, 4000 + 500 * j, 70 + j, N=32) for j in range(6)]
+    ref = []
+    for sc in scs:
+        e = make(sc)
+        e.advance(40)
+        e.set_option("derive_f", 0)
+        e.advance(40)
+        ref.append(e.download())
+        e.close()
+    engines = [make(sc) for sc in scs]
+    b = Batch(engines)
+    b.set_option("graph", graph)
+    b.advance(40)
+    for e in engines:
+        e.set_option("derive_f", 0)
+    b.advance(40)
+    outs = [e.download() for e in engines]
+    assert b.get_option("fused_eager_substeps") > 16
+    b.close()
+    for e, o, r in zip(engines, outs, ref):
+        for f in ("x", "v", "C", "F", "Jp"):
+            assert np.array_equal(o[f], r[f]), f
+        e.close()
+
+
 def test_batch_recaptures_after_a_change(gpu_lib):
     scs = small_batch()[:2]
     engines = [make(sc) for sc in scs]
