@@ -101,6 +101,7 @@ Sim::~Sim() {
   if (d_img_) (void)hipFree(d_img_);
   if (d_mxyz_) (void)hipFree(d_mxyz_);
   if (d_mkeys_) (void)hipFree(d_mkeys_);
+  if (d_rows_) (void)hipFree(d_rows_);
   for (int w = 0; w < kStageSlots; ++w) {
     if (h_stage_[w]) (void)hipHostFree(h_stage_[w]);
     if (stage_ev_[w]) (void)hipEventDestroy(stage_ev_[w]);
@@ -348,7 +349,7 @@ int Sim::ensure_capacity(int64_t n) {
   }
   cap_ = 0;
   for (int b = 0; b < 2; ++b) {
-    // (the planes; as rows with the materials and a flag behind them, download_soa)
+    // (the planes; as rows with the materials and a flag behind them, copy_scratch)
     HIPCHK(hipMalloc(&d_f_[b], sizeof(float) * (NUM_PLANES * cap + cap / 4 + 64)), "hipMalloc(particles)");
     HIPCHK(hipMalloc(&d_mat_[b], cap), "hipMalloc(material ids)");
     HIPCHK(hipMalloc(&d_id_[b], sizeof(uint32_t) * cap), "hipMalloc(particle ids)");
@@ -624,6 +625,35 @@ int Sim::remove(int64_t first, int64_t count, void* removed, hipStream_t s) {
   return MPM_OK;
 }
 
+// Scratch of calls that only read the state (downloads, meshes), which wait
+// for their work before they return. It is memory of its own: the particle copy
+// that the next reorder writes would do if every caller ordered the call
+// after the last advance, but beside an advance on a stream that it is not
+// ordered with it would overwrite the state, where the call should at worst
+// return a torn copy of it. (105 bytes a particle, made in the first such call,
+// 0.02 to 0.4 ms of it.) Where the device has no room for it, that copy is used
+// after all, behind everything that is on the device.
+int Sim::copy_scratch(size_t bytes, uint8_t** out) {
+  if (bytes > rows_cap_) {
+    if (d_rows_) (void)hipFree(d_rows_);
+    d_rows_ = nullptr;
+    rows_cap_ = 0;
+    if (hipMalloc((void**)&d_rows_, bytes) == hipSuccess) {
+      rows_cap_ = bytes;
+    } else {
+      (void)hipGetLastError();
+      d_rows_ = nullptr;
+    }
+  }
+  *out = d_rows_;
+  if (d_rows_) return MPM_OK;
+  if (bytes > sizeof(float) * (NUM_PLANES * (size_t)cap_ + (size_t)cap_ / 4 + 64))
+    return fail(MPM_ERR_CAPACITY, "no device memory for %zu bytes of scratch", bytes);
+  HIPCHK(hipDeviceSynchronize(), "hipDeviceSynchronize");
+  *out = (uint8_t*)d_f_[cur_ ^ 1];
+  return MPM_OK;
+}
+
 // The bytes pass through pinned slots, whose copies run at the link's rate
 // (about 50 GB/s here; straight into pageable memory they run at 10). Taking
 // a chunk out of its slot is the slow part: the caller's arrays are mostly
@@ -755,11 +785,14 @@ int Sim::mesh_build(int side, int radius, int64_t* ntri, hipStream_t s) {
     HIPCHK(hipMalloc(&d_mscratch_, sizeof(uint32_t) * (nc / 2048 + 2)), "hipMalloc(mesh scan)");
     mcube_cap_ = nc;
   }
-  // the bins use the rows' arrays before the rows do, and the particle copy
-  // that the next reorder overwrites
-  float* const other = d_f_[cur_ ^ 1];
-  const mpmk::MeshScratch w{d_mcount_, d_moff_, d_mscratch_, other ? (uint32_t*)(other + 3 * stride_) : nullptr,
-                            other, stride_};
+  // the bins use the rows' arrays before the rows do
+  uint8_t* pos = nullptr;
+  if (P_ > 0) {
+    const int rc = copy_scratch(sizeof(float) * 4 * (size_t)P_, &pos);
+    if (rc) return rc;
+  }
+  const mpmk::MeshScratch w{d_mcount_, d_moff_, d_mscratch_, pos ? (uint32_t*)pos + 3 * (size_t)P_ : nullptr,
+                            (float*)pos, (size_t)P_};
   const double fill = std::min(1.0, (double)std::max<int64_t>(1, occupied_) / (double)node_blocks());
   HIPCHK(mpmk::mesh_distance_field(particles(), side, vdx_f, cutoff, fill, w, d_sdf_, s), "mesh distance field");
   HIPCHK(mpmk::mesh_count(d_sdf_, side, rv, d_mcount_, s), "mesh count");
@@ -1264,8 +1297,8 @@ int Sim::advance(int32_t substeps, hipStream_t s) {
   return MPM_OK;
 }
 
-// The rows are put in original-index order on the device (k_export) in the
-// particle copy that the next reorder overwrites, then fetched as one range.
+// The rows are put in original-index order on the device (k_export), then
+// fetched as one range.
 // A pass over the planes on the host took 75 ms for 1,000,000 particles (an
 // id's 25 values from 25 planes); the device takes 0.1 ms and the fetch 3.
 int Sim::download_soa(float* x, float* v, float* C, float* F, float* Jp, uint8_t* mat,
@@ -1273,12 +1306,14 @@ int Sim::download_soa(float* x, float* v, float* C, float* F, float* Jp, uint8_t
   if (!uploaded_) return fail(MPM_ERR_STATE, "mpm_download_soa: nothing uploaded");
   const size_t n = (size_t)P_;
   if (n == 0) return MPM_OK;
-  float* const rows = d_f_[cur_ ^ 1];
-  uint8_t* const mats = (uint8_t*)(rows + (size_t)NUM_PLANES * n);
   const size_t bad_at = (sizeof(float) * NUM_PLANES * n + n + 3) & ~(size_t)3;
-  uint32_t* const bad = (uint32_t*)((uint8_t*)rows + bad_at);
+  uint8_t* rows = nullptr;
+  const int rs = copy_scratch(bad_at + 4, &rows);
+  if (rs) return rs;
+  uint8_t* const mats = rows + sizeof(float) * NUM_PLANES * n;
+  uint32_t* const bad = (uint32_t*)(rows + bad_at);
   HIPCHK(mpmk::fill_u32(bad, 1, 0u, s), "download flag");
-  HIPCHK(mpmk::export_state(particles(), rows, mats, bad, f_stale_ ? 1 : 0, s), "download order");
+  HIPCHK(mpmk::export_state(particles(), (float*)rows, mats, bad, f_stale_ ? 1 : 0, s), "download order");
   struct Piece { uint8_t* dst; size_t begin, bytes; };
   const Piece pieces[] = {
       {(uint8_t*)x, 4 * PL_X * n, 12 * n},    {(uint8_t*)v, 4 * PL_V * n, 12 * n},
@@ -1292,7 +1327,7 @@ int Sim::download_soa(float* x, float* v, float* C, float* F, float* Jp, uint8_t
     }
     if (off + len == bad_at + 4) std::memcpy(&corrupt, data + len - 4, 4);  // (chunks end at multiples of 4)
   };
-  const int rc = fetch_chunks((const uint8_t*)rows, bad_at + 4, take, s);
+  const int rc = fetch_chunks(rows, bad_at + 4, take, s);
   if (rc) return rc;
   if (corrupt) return fail(MPM_ERR_STATE, "mpm_download_soa: corrupt particle id");
   return MPM_OK;

@@ -179,6 +179,10 @@ class Sim {
   int upload_materials();
   int sort_particles(hipStream_t s);
   int substep(hipStream_t s);
+  // device scratch of a call that only reads the state and waits for its work
+  int copy_scratch(size_t bytes, uint8_t** out);
+  uint8_t* d_rows_ = nullptr;
+  size_t rows_cap_ = 0;
   // device bytes [0, bytes) to the host: `take` gets every chunk once it is in
   // pinned memory (offset, data, size), from several threads for large ones
   template <class Take>

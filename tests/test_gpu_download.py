@@ -6,7 +6,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from mpm_amd import MATERIAL_WC_LIQUID, Engine, Params, make_material
+from mpm_amd import MATERIAL_WC_LIQUID, Engine, MPMError, Params, make_material
 from mpm_amd._lib import check, lib
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +42,42 @@ def test_rows_come_back_in_upload_order(gpu_lib, n):
                                  mats.ctypes.data_as(C.POINTER(C.c_uint8)), None), eng.handle)
     assert np.array_equal(mats, mat) and np.array_equal(Jp, out["Jp"])
     eng.close()
+
+
+@pytest.mark.parametrize("reading", ["download", "save_state"])
+def test_reading_calls_leave_an_advance_in_flight_alone(gpu_lib, tmp_path, reading):
+    """Calls that read the state, on the null stream, while an advance runs on
+    a stream that they are not ordered with: what they return is torn (or
+    refused, where a particle's index is), the simulation is not."""
+    import torch
+
+    def scene():
+        rng = np.random.default_rng(3)
+        n = 60_000
+        e = Engine(Params(dt=1e-4, N=32))
+        e.set_materials([make_material(MATERIAL_WC_LIQUID, 1e-6, 1000.0, bulk_modulus=4e4)])
+        e.set_option("sort_every", 2)  # the particle copies change places often
+        v = rng.uniform(-1, 1, (n, 3)).astype(np.float32)
+        e.add_particles(rng.uniform(0.3, 0.7, (n, 3)).astype(np.float32), np.zeros(n, np.uint8), v=v)
+        e.upload()
+        return e
+
+    rounds, k = 6, 40
+    alone = scene()
+    alone.advance(rounds * k)
+    want = alone.download()
+    alone.close()
+    e = scene()
+    read = {"download": e.download, "save_state": lambda: e.save_state(str(tmp_path / "state"))}[reading]
+    stream = torch.cuda.Stream()  # does not wait for the null stream, nor that for it
+    for r in range(rounds):
+        e.advance(k, stream=stream)
+        try:
+            read()
+        except MPMError:
+            pass
+    stream.synchronize()
+    got = e.download()
+    e.close()
+    for f in ("x", "v", "C", "F", "Jp", "material"):
+        assert np.array_equal(got[f], want[f]), f
