@@ -788,11 +788,11 @@ int Sim::mesh_build(int side, int radius, int64_t* ntri, hipStream_t s) {
   // the bins use the rows' arrays before the rows do
   uint8_t* pos = nullptr;
   if (P_ > 0) {
-    const int rc = copy_scratch(sizeof(float) * 4 * (size_t)P_, &pos);
+    const int rc = copy_scratch(sizeof(float) * 5 * (size_t)P_, &pos);
     if (rc) return rc;
   }
-  const mpmk::MeshScratch w{d_mcount_, d_moff_, d_mscratch_, pos ? (uint32_t*)pos + 3 * (size_t)P_ : nullptr,
-                            (float*)pos, (size_t)P_};
+  uint32_t* const bins = (uint32_t*)pos + 3 * (size_t)P_;
+  const mpmk::MeshScratch w{d_mcount_, d_moff_, d_mscratch_, bins, bins + P_, (float*)pos, (size_t)P_};
   const double fill = std::min(1.0, (double)std::max<int64_t>(1, occupied_) / (double)node_blocks());
   HIPCHK(mpmk::mesh_distance_field(particles(), side, vdx_f, cutoff, fill, w, d_sdf_, s), "mesh distance field");
   HIPCHK(mpmk::mesh_count(d_sdf_, side, rv, d_mcount_, s), "mesh count");

@@ -230,12 +230,13 @@ hipError_t tile_combine(const TileSums& in, int64_t nblk, hipStream_t s);
 // vertices lie on, cube after cube) at the rows' scanned offsets (one more
 // entry than rows: the total).
 // Scratch of the field: mesh_bins(side)^3 counts, one start more, the scan's
-// tile sums (one per 2048 counts), a rank and 3 planes of pos_stride floats
-// for the particles.
+// tile sums (one per 2048 counts), and for the particles a bin, a rank and 3
+// planes of pos_stride floats.
 struct MeshScratch {
   uint32_t* count;
   uint32_t* start;
   uint32_t* scan;
+  uint32_t* bins;
   uint32_t* rank;
   float* pos;
   size_t pos_stride;

@@ -102,7 +102,7 @@ __device__ __forceinline__ size_t bin_of(const ParticlesDev& P, int64_t p, int s
 // hold its bin.
 __global__ void __launch_bounds__(256)
     k_bin_count(ParticlesDev P, int side, float vdx, int nb, uint32_t* __restrict__ count,
-                uint32_t* __restrict__ rank) {
+                uint32_t* __restrict__ bins, uint32_t* __restrict__ rank) {
   const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int lane = threadIdx.x & 63;
   const bool valid = p < P.n;
@@ -119,16 +119,20 @@ __global__ void __launch_bounds__(256)
   uint32_t base = 0;
   if (lane == first) base = atomicAdd(count + bin, (uint32_t)__popcll(mine));
   base = (uint32_t)__shfl((int)base, first);
+  bins[p] = bin;
   rank[p] = base + (uint32_t)__popcll(mine & ((1ull << lane) - 1ull));
 }
 
-// the positions in bin order, as 3 planes of `stride` floats
+// the positions in bin order, as 3 planes of `stride` floats. (The bin is the
+// one that was counted: found again from the position it could be another,
+// and its place past the arrays, if an advance that the caller did not order
+// with this call moves the particle in between.)
 __global__ void __launch_bounds__(256)
-    k_bin_scatter(ParticlesDev P, int side, float vdx, int nb, const uint32_t* __restrict__ start,
+    k_bin_scatter(ParticlesDev P, const uint32_t* __restrict__ start, const uint32_t* __restrict__ bins,
                   const uint32_t* __restrict__ rank, float* __restrict__ pos, size_t stride) {
   const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (p >= P.n) return;
-  const size_t at = start[bin_of(P, p, side, vdx, nb)] + rank[p];
+  const size_t at = start[bins[p]] + rank[p];
 #pragma unroll
   for (int a = 0; a < 3; ++a) pos[a * stride + at] = P.f[(PL_X + a) * P.stride + p];
 }
@@ -453,13 +457,13 @@ hipError_t mesh_distance_field(const ParticlesDev& P, int side, float vdx, float
     hipLaunchKernelGGL(k_sdf_scatter, gp, dim3(256), 0, s, P, side, vdx, cutoff, sdf);
     return hipGetLastError();
   }
-  if (!w.count || !w.start || !w.scan || !w.rank || w.pos_stride < (size_t)P.n) return hipErrorInvalidValue;
+  if (!w.count || !w.start || !w.scan || !w.bins || !w.rank || w.pos_stride < (size_t)P.n) return hipErrorInvalidValue;
   hipError_t e = fill_u32(w.count, bins, 0u, s);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_bin_count, gp, dim3(256), 0, s, P, side, vdx, nb, w.count, w.rank);
+  hipLaunchKernelGGL(k_bin_count, gp, dim3(256), 0, s, P, side, vdx, nb, w.count, w.bins, w.rank);
   e = exclusive_scan(w.count, w.start, bins, w.scan, w.start + bins, s);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_bin_scatter, gp, dim3(256), 0, s, P, side, vdx, nb, w.start, w.rank, w.pos, w.pos_stride);
+  hipLaunchKernelGGL(k_bin_scatter, gp, dim3(256), 0, s, P, w.start, w.bins, w.rank, w.pos, w.pos_stride);
   if (held < kGatherFew)
     hipLaunchKernelGGL(k_sdf_gather<1>, dim3((unsigned)((bins + 3) / 4)), dim3(256), 0, s, w.pos, w.pos_stride,
                        w.start, side, nb, vdx, cutoff, sdf);

@@ -44,7 +44,7 @@ def test_rows_come_back_in_upload_order(gpu_lib, n):
     eng.close()
 
 
-@pytest.mark.parametrize("reading", ["download", "save_state"])
+@pytest.mark.parametrize("reading", ["download", "mesh", "save_state"])
 def test_reading_calls_leave_an_advance_in_flight_alone(gpu_lib, tmp_path, reading):
     """Calls that read the state, on the null stream, while an advance runs on
     a stream that they are not ordered with: what they return is torn (or
@@ -68,7 +68,8 @@ def test_reading_calls_leave_an_advance_in_flight_alone(gpu_lib, tmp_path, readi
     want = alone.download()
     alone.close()
     e = scene()
-    read = {"download": e.download, "save_state": lambda: e.save_state(str(tmp_path / "state"))}[reading]
+    read = {"download": e.download, "mesh": lambda: e.mesh(48, 2),
+            "save_state": lambda: e.save_state(str(tmp_path / "state"))}[reading]
     stream = torch.cuda.Stream()  # does not wait for the null stream, nor that for it
     for r in range(rounds):
         e.advance(k, stream=stream)
