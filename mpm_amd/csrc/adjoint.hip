@@ -76,8 +76,8 @@ struct DiffK {
 
 // One axis of a particle's stencil: quadratic B-spline weights and their
 // derivatives (InterpolationKernel.cuh), node offsets and node indices. A node
-// outside the grid has weight 0 and the index of the nearest node inside,
-// which the stencil of a particle that reaches the grid has anyway.
+// outside the grid has weight 0 and the index of the nearest node inside, so
+// that a load of it is in range (plane_sums takes 0 for what it loads there).
 struct Axis {
   int base;
   int node[3];
@@ -86,12 +86,13 @@ struct Axis {
 
 struct Stencil {
   Axis ax[3];
-  bool outside;  // no node of the stencil in the grid: the particle is left as it is
+  bool clipped;  // a node of the stencil is not in the grid
+  bool outside;  // past the grid: the particle is left as it is
 };
 
 __device__ __forceinline__ Stencil make_stencil(const float x[3], const StepConsts& k) {
   Stencil s;
-  s.outside = false;
+  s.clipped = s.outside = false;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
     Axis& t = s.ax[a];
@@ -110,6 +111,7 @@ __device__ __forceinline__ Stencil make_stencil(const float x[3], const StepCons
       t.dp[i] = (float)node * k.dx - x[a];
       t.node[i] = min(max(node, 0), k.N - 1);
     }
+    s.clipped |= t.base < 0 || t.base > k.N - 3;
     s.outside |= t.base + 3 < 0 || t.base >= k.N;  // mpm.cu:31-35,129-133
   }
   return s;
@@ -251,6 +253,16 @@ __device__ __forceinline__ void plane_sums(const float4* __restrict__ grid, cons
 #pragma unroll
     for (int c = 0; c < 3; ++c)
       g[3 * b + c] = grid[((size_t)na * k.N + (size_t)ay.node[b]) * k.N + (size_t)az.node[c]];
+  if (__ballot(sn.clipped) != 0ull) {  // few wavefronts
+    // a weight of 0 would not do: it makes NaN of a value that is not finite
+    const auto in_grid = [&](int node) { return (unsigned)node < (unsigned)k.N; };
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        if (!(in_grid(sn.ax[0].base + plane) && in_grid(ay.base + b) && in_grid(az.base + c)))
+          g[3 * b + c] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
   if (UPDATE) {
 #pragma unroll
     for (int b = 0; b < 3; ++b)

@@ -140,3 +140,35 @@ def test_runs_of_substeps_with_and_without_tapes(gpu_lib, steps):
     heavy = b[0, :, 3] > 1e-6 * b[0, :, 3].max()  # (a vanishing mass's velocity is all rounding)
     assert off(a[0, heavy], b[0, heavy]) < 1e-4 and off(a[1, heavy], b[1, heavy]) < 1e-4
     assert torch.equal(a[0, :, 3] > 0, b[0, :, 3] > 0) and torch.equal(a[1, heavy][:, 3], b[1, heavy][:, 3])
+
+
+@pytest.mark.parametrize("where", ["below", "above"])
+def test_nodes_outside_the_grid_count_as_empty(gpu_lib, where):
+    """A stencil that reaches past a face skips the nodes there, and one of
+    which no node lies in the grid gets velocity 0, whatever the nodes at the
+    face hold: a particle whose momentum is infinite, or whose adjoint is,
+    leaves another one, which shares no node with it, alone."""
+    from mpm_amd.diff import DiffStepper, pack_state
+    dev = torch.device("cuda")
+    # x axis: base cells -3 and 0 (nodes 0..2), or N - 1 (node N - 1) and N - 4
+    a, b = ((-2.6, 0.7) if where == "below" else (N - 0.3, N - 3.2))
+    x = torch.tensor([[a / N, 0.5, 0.5], [b / N, 0.5, 0.5]])
+    F = torch.eye(3).expand(2, 3, 3)
+
+    def run(v, adj):
+        st = pack_state(x.to(dev), torch.tensor(v).to(dev), None, F.to(dev))
+        mu, lam = torch.full((2,), 1e3, device=dev), torch.full((2,), 1.5e3, device=dev)
+        s = DiffStepper(Params(dt=1e-4, N=N, gravity=-9.8, boundary=0.0, compat=COMPAT_FIXED), 1e-3, 1e-6, 2)
+        out, adj_in, tape = torch.empty_like(st), torch.empty_like(st), s.new_tape()
+        adj_out = torch.tensor(adj, device=dev).expand(24, 2).contiguous()
+        adj_mu, adj_lam = torch.zeros_like(mu), torch.zeros_like(lam)
+        s.forward(st, out, mu, lam, tape)
+        s.backward(st, mu, lam, tape, adj_out, adj_in, adj_mu, adj_lam)
+        return [t[..., 0].cpu() for t in (out, adj_in, adj_mu, adj_lam)]
+
+    v0 = [0.3, -0.2, 0.1]
+    want = run([v0, [0.0, 0.0, 0.0]], [1.0, 1.0])
+    assert all(torch.isfinite(t).all() for t in want)
+    for got in (run([v0, [float("inf")] * 3], [1.0, 1.0]), run([v0, [0.0] * 3], [1.0, float("inf")])):
+        for g, w in zip(got, want):
+            assert torch.equal(g, w), (g, w)
