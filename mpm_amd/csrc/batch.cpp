@@ -36,6 +36,7 @@
 #include <cstring>
 #include <cstdarg>
 #include <cstdio>
+#include <functional>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -43,6 +44,7 @@
 #include "../../include/mpm_hip.h"
 #include "engine.hpp"
 #include "kernels.hpp"
+#include "span.hpp"
 
 using mpm_engine::Sim;
 
@@ -70,7 +72,7 @@ struct mpm_batch_s {
   uint8_t* d_tables = nullptr;
   size_t tables_cap = 0;
   // argument tables of eager fused substeps: pinned slots used in turn, each
-  // with the event recorded after the substeps that last copied from it, and
+  // with the event recorded after the last copy from it, and
   // one device copy (the copies and launches are ordered on the origin stream)
   static constexpr int kEagerSlots = 2;
   uint8_t* h_eager[kEagerSlots] = {};
@@ -413,8 +415,8 @@ bool all_at_cycle_start(const mpm_batch_s* b, int* cycle);
 // the others' gaps and tails (a launch's last, partly occupied round of
 // workgroups). Either way the substeps' launches fork once and join once, so
 // the chains drift apart and one chain's grid update meets the other's fused
-// pass. Eager substeps are planned first, all their tables copied at once and
-// then launched: with a copy, a fork and a join for every substep, 42 substeps
+// pass. Eager substeps are planned first (span.hpp), all their tables copied at
+// once and then launched: with a copy, a fork and a join for every substep, 42 substeps
 // of 24 scenes (5,000 to 120,000 particles) took 9.4 ms, 16 at a time 8.7.
 int run_scenes_fused(mpm_batch_s* b, int32_t n, bool eager, int32_t* ran, size_t* recorded_bytes = nullptr) {
   const size_t nsc = b->scenes.size();
@@ -483,34 +485,48 @@ int run_scenes_fused(mpm_batch_s* b, int32_t n, bool eager, int32_t* ran, size_t
   b->eager_pending[slot] = false;
   tw = TableWriter{b, b->h_eager[slot], b->d_eager, b->eager_cap};
   std::vector<std::vector<Chain>> steps;
-  int cycle = 0;
+  struct Span {
+    mpm_batch_s* b;
+    std::function<int(int32_t)> plan, launch;
+    std::function<bool(int32_t)> more;
+    std::function<int()> begin, end;
+    std::vector<Sim::StepState> save() const {
+      std::vector<Sim::StepState> all;
+      for (const Sim* s : b->scenes) all.push_back(s->step_state());
+      return all;
+    }
+    void restore(const std::vector<Sim::StepState>& all) const {
+      for (size_t j = 0; j < all.size(); ++j) b->scenes[j]->set_step_state(all[j]);
+    }
+  } span{b};
+  span.plan = [&](int32_t) {
+    steps.emplace_back();
+    return plan(steps.back());
+  };
+  span.more = [&](int32_t planned) {
+    int cycle = 0;
+    return !(b->use_graph && all_at_cycle_start(b, &cycle) && n - planned >= cycle);
+  };
+  span.begin = [&]() -> int {
+    // (the device buffer is shared by the slots: the stream orders each copy
+    // after the kernels that read the last one)
+    if (tw.used) {
+      BCHK(hipMemcpyAsync(b->d_eager, b->h_eager[slot], tw.used, hipMemcpyHostToDevice, b->origin),
+           "hipMemcpyAsync(batch tables)");
+      BCHK(hipEventRecord(b->eager_ev[slot], b->origin), "hipEventRecord");
+      b->eager_pending[slot] = true;
+    }
+    return fork();
+  };
+  span.launch = [&](int32_t i) { return launch(steps[(size_t)i]); };
+  span.end = join;
   // Planning may enqueue work of its own on the chains' streams (a scene's F
   // planes written out): they wait for the origin before it, for the last
   // call's kernels, and again after the tables' copy.
   int rc = fork();
-  do {
-    steps.emplace_back();
-    if (!rc) rc = plan(steps.back());
-    if (rc) {
-      (void)join();
-      return rc;
-    }
-    *ran = (int32_t)steps.size();
-  } while (*ran < std::min<int32_t>(n, kEagerSpan) &&
-           !(b->use_graph && all_at_cycle_start(b, &cycle) && n - *ran >= cycle));
-  // (the device buffer is shared by the slots: the stream orders each copy
-  // after the kernels that read the last one)
-  if (tw.used)
-    BCHK(hipMemcpyAsync(b->d_eager, b->h_eager[slot], tw.used, hipMemcpyHostToDevice, b->origin),
-         "hipMemcpyAsync(batch tables)");
-  rc = fork();
-  for (size_t i = 0; i < steps.size() && !rc; ++i) rc = launch(steps[i]);
-  const int rj = join();
-  if (rc || rj) return rc ? rc : rj;
-  BCHK(hipEventRecord(b->eager_ev[slot], b->origin), "hipEventRecord");
-  b->eager_pending[slot] = true;
+  if (!rc) rc = mpm_engine::run_span(span, std::min<int32_t>(n, kEagerSpan), ran);
   b->eager_fused += *ran;
-  return MPM_OK;
+  return rc;
 }
 
 // Longest cycle recorded into one graph (substeps).

@@ -137,7 +137,7 @@ class Sim {
   }
   int sort_now(hipStream_t s) { return sort_particles(s); }
   // the same sort as arguments of the multi-scene sort kernels; sort_done()
-  // after they were launched
+  // once they are planned
   bool multi_sort_ok() const { return opt_.radix_bits == 8 && tiles_cap_ >= max_items(); }
   int sort_desc(mpmk::SortDesc& d);
   void sort_done() {
@@ -146,7 +146,7 @@ class Sim {
     items_valid_ = true;
   }
   // part 3: the fused pass (writes F planes out first on `s` if needed);
-  // fused_pass_done() after it was launched
+  // fused_pass_done() once it is planned
   int fused_pass(const float4* grid_v, int do_g2p, mpmk::ItemDesc& d, int& kinds, int64_t& launch,
                  hipStream_t s);
   void fused_pass_done(const mpmk::ItemDesc& d);
@@ -157,6 +157,30 @@ class Sim {
     grid_dead_ = true;
     ++steps_since_sort_;
     t_ += (double)prm_.dt;
+  }
+  // what the parts of a substep change on the host, to take it back where they
+  // were planned but not launched
+  struct StepState {
+    int cur, chunk, kinds;
+    bool pending_gather, items_valid, f_stale, grid_dead;
+    const float4* vel_grid;
+    int64_t steps_since_sort;
+    double t;
+  };
+  StepState step_state() const {
+    return {cur_, chunk_, kinds_, pending_gather_, items_valid_, f_stale_, grid_dead_, vel_grid_, steps_since_sort_, t_};
+  }
+  void set_step_state(const StepState& s) {
+    cur_ = s.cur;
+    chunk_ = s.chunk;
+    kinds_ = s.kinds;
+    pending_gather_ = s.pending_gather;
+    items_valid_ = s.items_valid;
+    f_stale_ = s.f_stale;
+    grid_dead_ = s.grid_dead;
+    vel_grid_ = s.vel_grid;
+    steps_since_sort_ = s.steps_since_sort;
+    t_ = s.t;
   }
   const float4* velocity_grid() const { return d_grid_[0]; }
   // every material is WC_LIQUID (the fused pass's liquid-only kernel)
