@@ -287,7 +287,10 @@ int mpm_load_state(mpm_handle h, const char* path);
  *                around the enqueue of each phase, for `rocprofv3
  *                --marker-trace`; host-side (when the launches were issued,
  *                not when the kernels ran). 0 (default): none
- * Results do not depend on the options beyond FP32 summation order. */
+ * Results do not depend on the options beyond FP32 summation order.
+ * Read only: "occupied_blocks", the blocks of 4^3 cells that held particles at
+ * the upload, with those of appended particles and less in proportion to
+ * removed ones; it sizes launches and picks the mesher's kernels. */
 int mpm_set_option(mpm_handle h, const char* name, int64_t value);
 int mpm_get_option(mpm_handle h, const char* name, int64_t* value);
 

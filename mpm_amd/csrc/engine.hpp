@@ -230,10 +230,13 @@ class Sim {
   bool f_canonical_ = false;
   bool f_stale_ = false;
   bool derives_f() const;
+  uint64_t staged_block(size_t i) const;
   bool dense_blocks(int64_t* occupied) const;  // from the staged particles
   bool use_mlp() const;
   bool dense_ = false;
-  int64_t occupied_ = 0;  // home blocks holding particles at the upload
+  // home blocks holding particles at the upload, an estimate after an append
+  // (their sum) or a removal (in proportion); sizes launches, picks kernels
+  int64_t occupied_ = 0;
   size_t staged_on_device_ = 0;  // staged particles the last upload / append copied
   // mesh buffers: distance field, per-row counts and offsets (or the bins'), scan scratch,
   // triangles; the last build's grid side and triangle count

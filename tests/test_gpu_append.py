@@ -142,3 +142,33 @@ def test_append_before_upload_is_an_error(gpu_lib):
     with pytest.raises(MPMError, match="nothing uploaded"):
         e.append()
     e.close()
+
+
+def test_occupied_blocks_follow_appends_and_removals(gpu_lib):
+    """The estimate that sizes launches and picks the mesher's kernels: the
+    blocks of an upload, those of appended particles added (at most all there
+    are), a share taken off with removed ones."""
+    sc = scenes.snow_spheres(n=20_000, N=32)
+    st = sc.state()
+    add = lambda e, part: e.add_particles(*(st[f][part] for f in ("x", "material", "v", "C", "F", "Jp")))
+    cells = np.clip(np.floor(st["x"] * np.float32(32)), 0, 31).astype(int) // 4
+    blocks = lambda part: len(np.unique(cells[part], axis=0))
+    e = engine(sc, slice(0, sc.n))
+    assert e.get_option("occupied_blocks") == blocks(slice(0, sc.n)) > 50
+    e.remove(0, sc.n // 2)
+    assert e.get_option("occupied_blocks") == blocks(slice(0, sc.n)) // 2
+    e.remove(0, sc.n // 2)
+    assert e.get_option("occupied_blocks") == 0
+    e.clear_particles()
+    add(e, slice(0, sc.n))
+    e.append()
+    assert e.get_option("occupied_blocks") == blocks(slice(0, sc.n))
+    e.close()
+    e = engine(sc, slice(0, 100))
+    for _ in range(9):
+        add(e, slice(100, sc.n))
+        e.append()
+    assert e.get_option("occupied_blocks") == min(8 ** 3, blocks(slice(0, 100)) + 9 * blocks(slice(100, sc.n)))
+    with pytest.raises(Exception, match="occupied_blocks"):
+        e.set_option("occupied_blocks", 1)
+    e.close()
