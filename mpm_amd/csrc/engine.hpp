@@ -211,12 +211,13 @@ class Sim {
   // pinned memory (offset, data, size), from several threads for large ones
   template <class Take>
   int fetch_chunks(const uint8_t* src, size_t bytes, const Take& take, hipStream_t s);
-  // pinned slots of fetch_chunks, each with the event of its last copy; at
-  // most kStageSlots of kStageBytes a handle
+  template <class Slot, class Take>
+  hipError_t fetch_through(const Slot* slot, size_t slots, size_t chunk, const uint8_t* src, size_t bytes,
+                           const Take& take, hipStream_t s);
+  // at most kStageSlots pinned slots of kStageBytes at a time, each with the
+  // event of its last copy
   static constexpr int kStageSlots = 8;
   static constexpr size_t kStageBytes = (size_t)2 << 20;
-  uint8_t* h_stage_[kStageSlots] = {};
-  size_t stage_bytes_[kStageSlots] = {};
   hipEvent_t stage_ev_[kStageSlots] = {};
   int hip_fail(hipError_t e, const char* what);
   int check_materials_cover_particles(const char* who);

@@ -82,3 +82,34 @@ def test_reading_calls_leave_an_advance_in_flight_alone(gpu_lib, tmp_path, readi
     e.close()
     for f in ("x", "v", "C", "F", "Jp", "material"):
         assert np.array_equal(got[f], want[f]), f
+
+
+def test_engines_download_from_several_threads(gpu_lib):
+    """Downloads share their pinned slots: those of six engines at a time, small
+    and large ones, each bring their own rows."""
+    import threading
+    rng = np.random.default_rng(5)
+    engines, xs = [], []
+    for n in (500, 20_000, 150_000, 700, 90_001, 150_000):
+        x = rng.uniform(0.2, 0.8, (n, 3)).astype(np.float32)
+        e = Engine(Params(dt=1e-4, N=24, gravity=0.0))
+        e.set_materials([make_material(MATERIAL_WC_LIQUID, 1e-6, 1000.0, bulk_modulus=4e4)])
+        e.add_particles(x, np.zeros(n, np.uint8))
+        e.upload()
+        engines.append(e)
+        xs.append(x)
+    bad = []
+
+    def work(e, x):
+        for _ in range(15):
+            if not np.array_equal(e.download()["x"], x):
+                bad.append(len(x))
+
+    threads = [threading.Thread(target=work, args=a) for a in zip(engines, xs)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    for e in engines:
+        e.close()
