@@ -116,6 +116,28 @@ def test_marching_cubes_matches_oracle(gpu_lib):
     assert np.array_equal(m["triangles"], tri)
 
 
+@pytest.mark.parametrize("side", [64, 65, 127, 130])
+def test_marching_cubes_over_several_stretches_of_a_row(gpu_lib, side):
+    """A wavefront takes the cubes of a row 63 at a time: one stretch, one cube
+    more, two full ones, three."""
+    from oracle.mesh import marching_cubes
+    N, r = 32, 2
+    rng = np.random.default_rng(side)
+    x = (0.03 + 0.94 * rng.random((1200, 3))).astype(np.float32)
+    e = engine_with(x, N)
+    m = e.mesh(side, r)
+    d = e.mesh_distance_field(side)
+    e.close()
+    _, _, iso = voxel_geometry(N, side, r)
+    vdx = float(N * np.float32(1.0 / N)) / side
+    tri, keys = marching_cubes(iso - d.astype(np.float64), vdx)
+    assert len(tri) > 10_000
+    last = (keys & np.uint64(0xffffffff)) % np.uint64(side)  # the edges' k: in the last stretch too
+    assert last.max() > 63 * ((side - 2) // 63)
+    assert np.array_equal(m["edges"], keys)
+    assert np.array_equal(m["triangles"], tri)
+
+
 def test_single_particle_sphere(gpu_lib):
     N, side, r = 32, 64, 6
     x = np.array([[0.50321, 0.4871, 0.51234]], np.float32)
