@@ -111,7 +111,7 @@ __device__ __forceinline__ Stencil make_stencil(const float x[3], const StepCons
       t.dp[i] = (float)node * k.dx - x[a];
       t.node[i] = min(max(node, 0), k.N - 1);
     }
-    s.clipped |= t.base < 0 || t.base > k.N - 3;
+    s.clipped |= (unsigned)t.base >= (unsigned)max(k.N - 2, 0);
     s.outside |= t.base + 3 < 0 || t.base >= k.N;  // mpm.cu:31-35,129-133
   }
   return s;
@@ -253,7 +253,7 @@ __device__ __forceinline__ void plane_sums(const float4* __restrict__ grid, cons
 #pragma unroll
     for (int c = 0; c < 3; ++c)
       g[3 * b + c] = grid[((size_t)na * k.N + (size_t)ay.node[b]) * k.N + (size_t)az.node[c]];
-  if (__ballot(sn.clipped) != 0ull) {  // few wavefronts
+  if (__builtin_expect(__ballot(sn.clipped) != 0ull, 0)) {
     // a weight of 0 would not do: it makes NaN of a value that is not finite
     const auto in_grid = [&](int node) { return (unsigned)node < (unsigned)k.N; };
 #pragma unroll
