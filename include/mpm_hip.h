@@ -471,12 +471,16 @@ int mpm_diff_substep_backward(const mpm_params* params, float particle_mass,
                               float* adj_lambda, float* grid, void* stream);
 
 /* A run of `steps` >= 1 differentiable substeps in one call: the kernels of
- * mpm_diff_substep, two launches per substep, all enqueued here. From
+ * mpm_diff_substep, one launch per substep after a clear and the first P2G,
+ * all enqueued here. From
  * state0, the state after substep j+1 goes to states + j*state_stride
  * (state_stride >= 24 n floats; state0 must not lie in that output) and its
- * grid tape to tapes + j*tape_stride (tape_stride a multiple of 4 >= 8 N^3 floats, or 0:
- * every substep writes the same tape, when no backward follows). grid: 4 N^3
- * floats of scratch. No reference counterpart. */
+ * grid tape to tapes + j*tape_stride (tape_stride a multiple of 4 >= 8 N^3
+ * floats, or 0: one tape for all, when no backward follows; it ends as the
+ * last substep's). Until the call's work is done every tape is scratch as well:
+ * a substep's momentum and mass sums lie in the next one's tape, or in the grid
+ * and the halves of the one tape in turn. grid: 4 N^3 floats of scratch, left
+ * with sums in it. No reference counterpart. */
 int mpm_diff_forward_steps(const mpm_params* params, float particle_mass, float particle_volume,
                            int64_t n, int32_t steps, const float* state0, float* states,
                            int64_t state_stride, const float* mu, const float* lambda, float* grid,

@@ -35,10 +35,17 @@
 // them (storing the state, the cells of the scatter, mu's adjoint).
 // A wavefront has its SIMD nearly to itself and runs its code once: short code
 // without branches, in which an LDS or memory round trip is waited for once, is
-// what counts. k_diff_step and k_adj_step took 26 and 38 us for 32,768
-// particles with one wavefront per 64 particles, now 12.2 and 13.6, the grid
-// update of 3 to 5 us in the first (2,197 particles: 19 and 29, now 9.6 and
-// 11.4). The SVD's serial chain is 2 us of each. Newton's iteration for the
+// what counts. For a jittered cube of 32,768 particles under shear
+// (perf/cases.py's rollouts) k_diff_step and k_adj_step took 26 and 38 us with
+// one wavefront per 64 particles, now 12.4 and 13.6, the grid update of 3 to 5 us
+// in the first (2,197 particles: 19 and 29, now 9.6 and 11.4); for bench.py's
+// cube, which falls freely in lattice order, 18.8 and 29.8, now 11.4 and 12.4.
+// Where the chip is full the wavefronts' repeated work still costs less than the
+// shorter chain saves: a substep forward and its adjoint 77 + 104 -> 56 + 80 us for
+// 262,144 particles in cell order, 541 + 690 -> 374 + 580 for 2,097,152. (In
+// random order the atomics bound both: 91 + 98 -> 79 + 82 us for 32,768, 284 + 379
+// -> 311 + 327 for 262,144 on 64^3, 1,149 + 1,150 -> 1,068 + 1,063 for 1,000,000.)
+// The SVD's serial chain is 2 us of each launch. Newton's iteration for the
 // rotation takes 0.6, but the position's adjoint is what is left of momenta
 // that cancel: the last bits by which the rotations differ come out as 1e-3 of
 // its root mean square in sparse cells.

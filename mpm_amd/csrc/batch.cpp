@@ -212,7 +212,7 @@ constexpr int32_t kEagerSpan = 16;  // eager substeps planned and launched toget
 
 // table bytes of one substep at most: per chain (four at most) a reduce
 // table, up to two pass tables and a sort table, each launch with its prefix
-// (the sort: about 20 launches), every table 256-byte aligned
+// (the sort: 6, and 3 for each of at most 3 digit passes), every table 256-byte aligned
 size_t tables_per_substep(size_t ns) {
   return ns * (sizeof(mpmk::ReduceDesc) + 2 * sizeof(mpmk::ItemDesc) + sizeof(mpmk::SortDesc)) +
          112 * (4 * (ns + 1) + 256) + 4 * 256;
