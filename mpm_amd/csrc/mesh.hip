@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W)
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6, turn = W == 1 ? 0 : wave;
   const uint32_t unb = (uint32_t)nb;  // (at most 256^3 blocks)
-  const uint32_t blk = W == 1 ? blockIdx.x * 4u + (uint32_t)wave : blockIdx.x;
+  const uint32_t blk = W == 1 ? blockIdx.x * 4u + (uint32_t)wave : blockIdx.y * (unb * unb) + blockIdx.x;
   if (blk >= unb * unb * unb) return;  // uniform for the wavefront (W = 1), else for the workgroup
   __shared__ uint32_t bound;
   __shared__ float least[W == 1 ? 1 : W][64];
@@ -467,12 +467,16 @@ hipError_t mesh_distance_field(const ParticlesDev& P, int side, float vdx, float
   if (held < kGatherFew)
     hipLaunchKernelGGL(k_sdf_gather<1>, dim3((unsigned)((bins + 3) / 4)), dim3(256), 0, s, w.pos, w.pos_stride,
                        w.start, side, nb, vdx, cutoff, sdf);
-  else if (held < kGatherMany)
-    hipLaunchKernelGGL(k_sdf_gather<4>, dim3((unsigned)bins), dim3(256), 0, s, w.pos, w.pos_stride, w.start, side,
-                       nb, vdx, cutoff, sdf);
-  else
-    hipLaunchKernelGGL(k_sdf_gather<16>, dim3((unsigned)bins), dim3(1024), 0, s, w.pos, w.pos_stride, w.start, side,
-                       nb, vdx, cutoff, sdf);
+  else {
+    // (by planes of blocks: a dimension of a launch has less than 2^32 threads, and
+    // 1024 for each of the blocks of 700^3 voxels are more)
+    const dim3 g((unsigned)nb * (unsigned)nb, (unsigned)nb);
+    if (held < kGatherMany)
+      hipLaunchKernelGGL(k_sdf_gather<4>, g, dim3(256), 0, s, w.pos, w.pos_stride, w.start, side, nb, vdx, cutoff, sdf);
+    else
+      hipLaunchKernelGGL(k_sdf_gather<16>, g, dim3(1024), 0, s, w.pos, w.pos_stride, w.start, side, nb, vdx, cutoff,
+                         sdf);
+  }
   return hipGetLastError();
 }
 

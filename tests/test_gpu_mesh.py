@@ -232,3 +232,38 @@ def test_mesh_errors_and_empty_set(gpu_lib):
         e.mesh_distance_field(16)
     assert np.all(e.mesh_distance_field(32) == voxel_geometry(32, 32, 2)[1])
     e.close()
+
+
+def test_distance_field_of_a_crowded_body_on_a_fine_grid(gpu_lib):
+    """Thousands of particles in a block of voxels and 5,400,000 blocks: 16
+    wavefronts for each of them. Sampled voxels, against the distance to the
+    nearest particle in float32 (away from the cut-off, where the truncated box
+    decides), and no voxel left out."""
+    N, side, r, n = 128, 700, 8, 300_000
+    rng = np.random.default_rng(11)
+    x = ((64 + 3.9 * rng.random((n, 3))) / 128).astype(np.float32)  # one block of 4^3 cells
+    e = engine_with(x, N)
+    assert e.get_option("occupied_blocks") == 1
+    e.mesh(side, r)
+    got = e.mesh_distance_field(side)
+    e.close()
+    vdx, cutoff, _ = voxel_geometry(N, side, r)
+    vdx, cutoff = np.float32(vdx), np.float32(cutoff)
+    assert got.max() == cutoff and got.min() >= 0  # (every voxel written)
+    lo, hi = int(0.5 * side) - r - 6, int(0.54 * side) + r + 6
+    outside = np.ones(got.shape, bool)
+    outside[lo:hi, lo:hi, lo:hi] = False
+    assert (got[outside] == cutoff).all()
+    v = rng.integers(lo, hi, (600, 3))
+    node = v.astype(np.float32) * vdx
+    d = np.full(len(v), np.inf, np.float32)
+    for part in np.array_split(x, 20):
+        q = part[None] - node[:, None]
+        q = q * q
+        d = np.minimum(d, (q[..., 0] + (q[..., 1] + q[..., 2])).min(1))
+    d = np.minimum(np.sqrt(d), cutoff)
+    clear = np.abs(d - cutoff) > 0.01 * cutoff
+    clear |= d == cutoff
+    g = got[v[:, 0], v[:, 1], v[:, 2]]
+    assert clear.sum() > 500 and np.array_equal(g[clear & (d < cutoff)], d[clear & (d < cutoff)])
+    assert (g[clear & (d == cutoff)] >= np.float32(0.98) * cutoff).all()
