@@ -92,7 +92,7 @@ struct PinnedMemory {
   }
   static void drop(uint8_t* p) { (void)hipHostFree(p); }
 };
-using PinnedPool = SlotPool<PinnedMemory, 16>;
+using PinnedPool = SlotPool<PinnedMemory, 16, ((size_t)512 << 10)>;
 static PinnedPool& pinned_pool() {
   static PinnedPool& pool = *new PinnedPool;  // (no destructor at exit, where the runtime may be gone)
   return pool;
@@ -662,11 +662,14 @@ int Sim::remove(int64_t first, int64_t count, void* removed, hipStream_t s) {
 // after all, behind everything that is on the device.
 int Sim::copy_scratch(size_t bytes, uint8_t** out) {
   if (bytes > rows_cap_) {
+    // (room to grow from the second time on: a scene that gets particles for
+    // every frame would have it made for every download)
+    const size_t want = rows_cap_ ? bytes + bytes / 2 : bytes;
     if (d_rows_) (void)hipFree(d_rows_);
     d_rows_ = nullptr;
     rows_cap_ = 0;
-    if (hipMalloc((void**)&d_rows_, bytes) == hipSuccess) {
-      rows_cap_ = bytes;
+    if (hipMalloc((void**)&d_rows_, want) == hipSuccess) {
+      rows_cap_ = want;
     } else {
       (void)hipGetLastError();
       d_rows_ = nullptr;

@@ -15,7 +15,9 @@
 namespace mpm_engine {
 
 // Memory: static uint8_t* make(size_t bytes) (null: none left), drop(uint8_t*).
-template <class Memory, size_t kMax>
+// Blocks are made in steps of kStep bytes, so that calls whose size grows by
+// little use one again.
+template <class Memory, size_t kMax, size_t kStep>
 class SlotPool {
  public:
   struct Slot {
@@ -68,7 +70,8 @@ class SlotPool {
     return made_ < kMax;
   }
   bool new_block(size_t bytes, Slot* out) {
-    *out = {Memory::make(bytes), bytes};
+    const size_t size = (bytes + kStep - 1) / kStep * kStep;
+    *out = {Memory::make(size), size};
     if (out->p) ++made_;
     return out->p != nullptr;
   }

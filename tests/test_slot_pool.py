@@ -28,7 +28,7 @@ struct Memory {
   }
   static void drop(uint8_t* p) { --live; std::free(p); }
 };
-using Pool = mpm_engine::SlotPool<Memory, 4>;
+using Pool = mpm_engine::SlotPool<Memory, 4, 32>;
 #define CHECK(c) if (!(c)) { std::printf("line %d: %s (live %d, made %d)\n", __LINE__, #c, (int)live, (int)made); std::exit(1); }
 
 int main() {
@@ -54,6 +54,14 @@ int main() {
   CHECK(live == 4);
   pool.detach();
   CHECK(live == 0);                                 // the last user gives all back
+  made = 0;
+  pool.attach();
+  for (size_t bytes = 1000; bytes < 1064; ++bytes) {  // a call that grows: one block for every 32 bytes more
+    CHECK(pool.take(1, bytes, a) == 1 && a[0].bytes >= bytes);
+    pool.give(a, 1);
+  }
+  CHECK(made == 3 && live == 3);
+  pool.detach();
   none_left = true;
   CHECK(pool.take(2, 10, a) == 0);
   none_left = false;
