@@ -55,6 +55,7 @@
 // Fbar += 2 U N V^T, N_ij = M_ij / (s_i + s_j).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "device_math.hpp"
@@ -73,6 +74,11 @@ constexpr int kThreads = 4 * kWave;  // fourth for what does not wait for the pl
 constexpr int kNodes = 27;           // of a stencil
 constexpr int kRunsAhead = 8;        // runs whose sums are loaded together
 constexpr int kNowhere = 1 << 20;    // a cell that no node is next to
+// Workgroups of a launch at most, in 2^30 threads: a dimension of a launch has
+// less than 2^32, and more wrap around without an error (1,073,741,824
+// particles; 1024^3 nodes are 2^22 workgroups by themselves). Kernels get the
+// number of their launch's first one.
+constexpr unsigned kMaxBlocks = 1u << 22;
 
 struct DiffK {
   StepConsts k;
@@ -598,7 +604,8 @@ __device__ __forceinline__ void node_block(const NodeWork& w, const DiffK& d, un
 // G2P of substep n from `st` into `out` (particles outside the grid are
 // copied), fused with the P2G of substep n+1 of the new state into `grid`.
 // Without G2P: the P2G of `st`. Without P2G: the G2P only. The first `blocks`
-// workgroups hold the particles, those past them the nodes.
+// workgroups hold the particles, those past them the nodes; `first` is the
+// launch's first one.
 // The G2P updates the nodes that it gathers by itself, from substep n's sums: 27
 // times as many updates as there are nodes, for 0.95 us of 12.2 (32,768
 // particles), where the grid update as a launch of its own took 3.3 us, a gap
@@ -607,17 +614,18 @@ template <bool G2P, bool P2G>
 __global__ void __launch_bounds__(kThreads)
     k_diff_step(const float* __restrict__ st, float* __restrict__ out, const float4* __restrict__ sums,
                 const float* __restrict__ mu, const float* __restrict__ lam, DiffK d,
-                float* __restrict__ grid, unsigned blocks, NodeWork nodes) {
+                float* __restrict__ grid, unsigned blocks, NodeWork nodes, unsigned first) {
   __shared__ float4 part[G2P ? kPlanes * 3 * kWave : 1];
   __shared__ ScatterShared sh;  // (unused without P2G, then it takes no LDS)
   const StepConsts& k = d.k;
-  if (blockIdx.x >= blocks) {
-    node_block(nodes, d, blockIdx.x - blocks);
+  const unsigned block = first + blockIdx.x;
+  if (block >= blocks) {
+    node_block(nodes, d, block - blocks);
     return;
   }
   const int lane = threadIdx.x & (kWave - 1);
   const int plane = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t p = (int64_t)blockIdx.x * kWave + lane, n = d.n;
+  const int64_t p = (int64_t)block * kWave + lane, n = d.n;
   const bool valid = p < n;
   float x[3] = {0.f, 0.f, 0.f}, v[3] = {0.f, 0.f, 0.f}, C[9], F[9];
 #pragma unroll
@@ -724,13 +732,13 @@ __global__ void __launch_bounds__(kThreads)
     k_adj_step(const float* __restrict__ st_s, const float* __restrict__ mu, const float* __restrict__ lam,
                const float4* __restrict__ gm, const float* adj_src, const float* __restrict__ st_prev,
                const float4* __restrict__ vel_prev, float* adj_dst, float* __restrict__ adj_mu,
-               float* __restrict__ adj_lam, float* __restrict__ gv_out, DiffK d) {
+               float* __restrict__ adj_lam, float* __restrict__ gv_out, DiffK d, unsigned first) {
   __shared__ float4 part_p[P2GA ? kPlanes * 4 * kWave : 1];
   __shared__ float4 part_g[G2PA ? kPlanes * 4 * kWave : 1];
   __shared__ ScatterShared sh;  // (unused without G2PA)
   const int lane = threadIdx.x & (kWave - 1);
   const int plane = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t p = (int64_t)blockIdx.x * kWave + lane, n = d.n;
+  const int64_t p = (int64_t)(first + blockIdx.x) * kWave + lane, n = d.n;
   const StepConsts& k = d.k;
   const bool valid = p < n;
   // adjoint of X_s
@@ -982,6 +990,12 @@ size_t nodes_of(const StepConsts& k) { return (size_t)k.N * k.N * k.N; }
 unsigned node_blocks(const StepConsts& k) { return (unsigned)((nodes_of(k) + 255) / 256); }
 unsigned particle_blocks(int64_t n) { return (unsigned)((n + kWave - 1) / kWave); }
 
+// launch(workgroups, first one) for all of `blocks`
+template <class Launch>
+void launch_blocks(unsigned blocks, const Launch& launch) {
+  for (unsigned first = 0; first < blocks; first += kMaxBlocks) launch(dim3(std::min(blocks - first, kMaxBlocks)), first);
+}
+
 // the two halves of a tape slot: velocities (read by G2P), then the rest
 const float4* tape_v(const float* tape) { return reinterpret_cast<const float4*>(tape); }
 const float4* tape_w(const float* tape, const StepConsts& k) {
@@ -1063,22 +1077,24 @@ hipError_t diff_forward_steps(const StepConsts& k, float mass, float volume, int
   hipLaunchKernelGGL(k_zero4, dim3(gn), dim3(256), 0, s, sums(0), nodes_of(k));
   if (n > 0 || steps > 1) {
     const NodeWork w = {nullptr, nullptr, nullptr, sums(1)};
-    hipLaunchKernelGGL((k_diff_step<false, true>), dim3(gp + (steps > 1 ? gn : 0u)), dim3(kThreads), 0, s, st0,
-                       (float*)nullptr, (const float4*)nullptr, mu, lam, d, (float*)sums(0), gp, w);
+    launch_blocks(gp + (steps > 1 ? gn : 0u), [&](dim3 g, unsigned first) {
+      hipLaunchKernelGGL((k_diff_step<false, true>), g, dim3(kThreads), 0, s, st0, (float*)nullptr,
+                         (const float4*)nullptr, mu, lam, d, (float*)sums(0), gp, w, first);
+    });
   }
   for (int32_t j = 0; j < steps; ++j) {
     const float* in = j == 0 ? st0 : states + (size_t)(j - 1) * (size_t)state_stride;
     float* out = states + (size_t)j * (size_t)state_stride;
     const bool last = j + 1 == steps, taped = last || tape_stride > 0;
     const NodeWork w = {sums(j), taped ? tape_v(tape(j)) : nullptr, taped ? tape_w(tape(j), k) : nullptr, sums(j + 2)};
-    const unsigned blocks = gp + (w.tv || w.clear ? gn : 0u);
-    if (blocks == 0) continue;
-    if (!last)
-      hipLaunchKernelGGL((k_diff_step<true, true>), dim3(blocks), dim3(kThreads), 0, s, in, out, (const float4*)w.sums,
-                         mu, lam, d, (float*)sums(j + 1), gp, w);
-    else
-      hipLaunchKernelGGL((k_diff_step<true, false>), dim3(blocks), dim3(kThreads), 0, s, in, out, (const float4*)w.sums,
-                         mu, lam, d, (float*)nullptr, gp, w);
+    launch_blocks(gp + (w.tv || w.clear ? gn : 0u), [&](dim3 g, unsigned first) {
+      if (!last)
+        hipLaunchKernelGGL((k_diff_step<true, true>), g, dim3(kThreads), 0, s, in, out, (const float4*)w.sums, mu, lam,
+                           d, (float*)sums(j + 1), gp, w, first);
+      else
+        hipLaunchKernelGGL((k_diff_step<true, false>), g, dim3(kThreads), 0, s, in, out, (const float4*)w.sums, mu, lam,
+                           d, (float*)nullptr, gp, w, first);
+    });
   }
   return hipGetLastError();
 }
@@ -1103,26 +1119,30 @@ hipError_t diff_backward_steps(const StepConsts& k, float mass, float volume, in
   auto tape = [&](int32_t j) { return tapes + (size_t)j * (size_t)tape_stride; };
   hipLaunchKernelGGL(k_zero4, dim3(gn), dim3(256), 0, s, ga, nodes);
   // the G2P adjoint of the last substep, from the caller's adjoint
-  if (n > 0)
-    hipLaunchKernelGGL((k_adj_step<false, true>), dim3(gp), dim3(kThreads), 0, s, (const float*)nullptr,
-                       (const float*)nullptr, (const float*)nullptr, (const float4*)nullptr, adj_out,
-                       state(steps - 1), tape_v(tape(steps - 1)), work, (float*)nullptr, (float*)nullptr,
-                       (float*)ga, d);
+  launch_blocks(gp, [&](dim3 g, unsigned first) {
+    hipLaunchKernelGGL((k_adj_step<false, true>), g, dim3(kThreads), 0, s, (const float*)nullptr, (const float*)nullptr,
+                       (const float*)nullptr, (const float4*)nullptr, adj_out, state(steps - 1),
+                       tape_v(tape(steps - 1)), work, (float*)nullptr, (float*)nullptr, (float*)ga, d, first);
+  });
   for (int32_t j = steps - 1; j >= 0; --j) {
     hipLaunchKernelGGL(k_adj_grid, dim3(gn), dim3(256), 0, s, ga, j > 0 ? gb : (float4*)nullptr,
                        tape_v(tape(j)), tape_w(tape(j), k), k);
     if (n == 0) continue;
     if (j > 0) {
-      hipLaunchKernelGGL((k_adj_step<true, true>), dim3(gp), dim3(kThreads), 0, s, state(j), mu, lam,
-                         (const float4*)ga, (const float*)work, state(j - 1), tape_v(tape(j - 1)), work, adj_mu,
-                         adj_lam, (float*)gb, d);
+      launch_blocks(gp, [&](dim3 g, unsigned first) {
+        hipLaunchKernelGGL((k_adj_step<true, true>), g, dim3(kThreads), 0, s, state(j), mu, lam, (const float4*)ga,
+                           (const float*)work, state(j - 1), tape_v(tape(j - 1)), work, adj_mu, adj_lam, (float*)gb, d,
+                           first);
+      });
       float4* t = ga;
       ga = gb;
       gb = t;
     } else {
-      hipLaunchKernelGGL((k_adj_step<true, false>), dim3(gp), dim3(kThreads), 0, s, state(0), mu, lam,
-                         (const float4*)ga, (const float*)work, (const float*)nullptr, (const float4*)nullptr,
-                         adj_in, adj_mu, adj_lam, (float*)nullptr, d);
+      launch_blocks(gp, [&](dim3 g, unsigned first) {
+        hipLaunchKernelGGL((k_adj_step<true, false>), g, dim3(kThreads), 0, s, state(0), mu, lam, (const float4*)ga,
+                           (const float*)work, (const float*)nullptr, (const float4*)nullptr, adj_in, adj_mu, adj_lam,
+                           (float*)nullptr, d, first);
+      });
     }
   }
   return hipGetLastError();

@@ -172,3 +172,53 @@ def test_nodes_outside_the_grid_count_as_empty(gpu_lib, where):
     for got in (run([v0, [float("inf")] * 3], [1.0, 1.0]), run([v0, [0.0] * 3], [1.0, float("inf")])):
         for g, w in zip(got, want):
             assert torch.equal(g, w), (g, w)
+
+
+def test_the_largest_grid(gpu_lib):
+    """1024^3 nodes, whose workgroups and the particles' take two launches: the
+    step of a 16^3 grid at the upper corner, scaled by powers of two. Lengths
+    are 1/64, so velocities, gravity and momenta are, and the stress's share
+    with volume / 64^2; offsets and weights are the same bits, the positions'
+    rounding is not. Tolerances as above."""
+    from mpm_amd.diff import DiffStepper, pack_state
+    dev = torch.device("cuda")
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("48 GiB of grids")
+    n, rng = 3000, np.random.default_rng(1)
+    X = np.round(rng.uniform(5.0, 14.4, (n, 3)) * 1024) / 1024  # in cells
+    v = rng.uniform(-1, 1, (n, 3)).astype(np.float32)
+    C = rng.uniform(-5, 5, (n, 3, 3)).astype(np.float32)
+    F = deformations("small", rng, n).astype(np.float32)
+    adj = rng.standard_normal((24, n)).astype(np.float32)
+
+    def run(grid, scale):
+        x = ((grid - 16 + X) / grid).astype(np.float32)
+        t = [torch.from_numpy(a).to(dev) for a in (x, v * np.float32(scale), C, F)]
+        st = pack_state(*t)
+        mu, lam = torch.full((n,), 1e3, device=dev), torch.full((n,), 1.5e3, device=dev)
+        s = DiffStepper(Params(dt=1e-4, N=grid, gravity=-9.8 * scale, boundary=0.0, compat=COMPAT_FIXED), 1e-3,
+                        1e-6 * scale * scale, n)
+        out, adj_in, tape = torch.empty_like(st), torch.empty_like(st), s.new_tape()
+        a = torch.from_numpy(adj).to(dev)
+        a[0:6] /= scale  # the adjoints of lengths and velocities
+        adj_mu, adj_lam = torch.zeros_like(mu), torch.zeros_like(lam)
+        s.forward(st, out, mu, lam, tape)
+        s.backward(st, mu, lam, tape, a.contiguous(), adj_in, adj_mu, adj_lam)
+        moved = (out[0:3] - st[0:3]) / scale
+        fwd = [moved, out[3:6] / scale, out[6:15], out[15:24]]
+        back = [adj_in[0:3] * scale, adj_in[3:6] * scale, adj_in[6:15], adj_in[15:24], adj_mu, adj_lam]
+        return [f.double().cpu() for f in fwd], [b.double().cpu() for b in back]
+
+    small = run(16, 1.0)
+    large = run(1024, 1.0 / 64)
+    torch.cuda.empty_cache()
+
+    def off(a, b):
+        return float((a - b).norm() / b.norm())
+
+    for k, (a, b) in enumerate(zip(large[0][1:], small[0][1:])):
+        assert off(a, b) < 1e-4, (k, off(a, b))
+    assert float((large[0][0] - small[0][0]).abs().max()) < 64 * 1.2e-7  # (two ulps below 1, scaled)
+    for k, (a, b) in enumerate(zip(large[1], small[1])):
+        assert off(a, b) < 1e-3, (k, off(a, b))
