@@ -88,12 +88,24 @@ __device__ __forceinline__ int voxel_of(float x, float vdx, int side) {  // clam
   return max(0, min(side - 1, (int)(x / vdx)));
 }
 
-// bin of 4^3 voxels that holds particle p
-__device__ __forceinline__ size_t bin_of(const ParticlesDev& P, int64_t p, int side, float vdx, int nb) {
+constexpr uint32_t kNoBin = 0xffffffffu;
+
+// Bin of 4^3 voxels that holds particle p, the nearest one for a particle past
+// the grid; none for one too far off to matter (the hundredth is for rounding),
+// or whose position is not a number: a simulation that has come apart would
+// crowd the bins at the faces with them (half of 1,000,000 particles: 60 ms).
+__device__ __forceinline__ uint32_t bin_of(const ParticlesDev& P, int64_t p, int side, float vdx, float cutoff,
+                                           int nb) {
+  const float lo = -1.01f * cutoff, hi = (float)(side - 1) * vdx - lo;
   int b[3];
+  bool near = true;
 #pragma unroll
-  for (int a = 0; a < 3; ++a) b[a] = voxel_of(P.f[(PL_X + a) * P.stride + p], vdx, side) / kBinEdge;
-  return ((size_t)b[0] * nb + b[1]) * nb + b[2];
+  for (int a = 0; a < 3; ++a) {
+    const float x = P.f[(PL_X + a) * P.stride + p];
+    near = near && x >= lo && x <= hi;
+    b[a] = voxel_of(x, vdx, side) / kBinEdge;
+  }
+  return near ? (uint32_t)((b[0] * nb + b[1]) * nb + b[2]) : kNoBin;  // (at most 256^3 bins)
 }
 
 // Neighbouring particles mostly share bins (they are in cell order), and the
@@ -101,12 +113,13 @@ __device__ __forceinline__ size_t bin_of(const ParticlesDev& P, int64_t p, int s
 // particles in 50 bins): one lane adds for all lanes of its wavefront that
 // hold its bin.
 __global__ void __launch_bounds__(256)
-    k_bin_count(ParticlesDev P, int side, float vdx, int nb, uint32_t* __restrict__ count,
+    k_bin_count(ParticlesDev P, int side, float vdx, float cutoff, int nb, uint32_t* __restrict__ count,
                 uint32_t* __restrict__ bins, uint32_t* __restrict__ rank) {
   const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int lane = threadIdx.x & 63;
-  const bool valid = p < P.n;
-  const uint32_t bin = valid ? (uint32_t)bin_of(P, p, side, vdx, nb) : 0u;  // (at most 256^3)
+  const uint32_t bin = p < P.n ? bin_of(P, p, side, vdx, cutoff, nb) : kNoBin;
+  const bool valid = bin != kNoBin;
+  if (p < P.n) bins[p] = bin;
   uint64_t mine = 0ull, left = __ballot(valid);
   while (left) {
     const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)bin, __ffsll((long long)left) - 1);
@@ -119,7 +132,6 @@ __global__ void __launch_bounds__(256)
   uint32_t base = 0;
   if (lane == first) base = atomicAdd(count + bin, (uint32_t)__popcll(mine));
   base = (uint32_t)__shfl((int)base, first);
-  bins[p] = bin;
   rank[p] = base + (uint32_t)__popcll(mine & ((1ull << lane) - 1ull));
 }
 
@@ -132,7 +144,9 @@ __global__ void __launch_bounds__(256)
                   const uint32_t* __restrict__ rank, float* __restrict__ pos, size_t stride) {
   const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (p >= P.n) return;
-  const size_t at = start[bins[p]] + rank[p];
+  const uint32_t bin = bins[p];
+  if (bin == kNoBin) return;
+  const size_t at = start[bin] + rank[p];
 #pragma unroll
   for (int a = 0; a < 3; ++a) pos[a * stride + at] = P.f[(PL_X + a) * P.stride + p];
 }
@@ -460,7 +474,7 @@ hipError_t mesh_distance_field(const ParticlesDev& P, int side, float vdx, float
   if (!w.count || !w.start || !w.scan || !w.bins || !w.rank || w.pos_stride < (size_t)P.n) return hipErrorInvalidValue;
   hipError_t e = fill_u32(w.count, bins, 0u, s);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_bin_count, gp, dim3(256), 0, s, P, side, vdx, nb, w.count, w.bins, w.rank);
+  hipLaunchKernelGGL(k_bin_count, gp, dim3(256), 0, s, P, side, vdx, cutoff, nb, w.count, w.bins, w.rank);
   e = exclusive_scan(w.count, w.start, bins, w.scan, w.start + bins, s);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_bin_scatter, gp, dim3(256), 0, s, P, w.start, w.bins, w.rank, w.pos, w.pos_stride);

@@ -234,6 +234,28 @@ def test_mesh_errors_and_empty_set(gpu_lib):
     e.close()
 
 
+@pytest.mark.parametrize("side,r", [(60, 3), (50, 5)])
+def test_distance_field_of_a_scene_that_came_apart(gpu_lib, side, r):
+    """Positions that are no numbers, infinite, far past the box, or about the
+    cut-off's distance past it, among ordinary ones: the oracle's field."""
+    N, n = 24, 4000
+    rng = np.random.default_rng(side)
+    x = rng.uniform(0.05, 0.95, (n, 3))
+    cut = (r + 1) / side
+    odd = [np.nan, np.inf, -np.inf, 1e30, -1e30, -5.0, 7.0, -cut, -0.999 * cut, -1.005 * cut, -1.02 * cut,
+           1 - 1 / side + cut, 1 - 1 / side + 0.999 * cut, 1 - 1 / side + 1.02 * cut]
+    for i in range(2000):
+        x[i, rng.integers(3)] = odd[i % len(odd)]
+    x = x.astype(np.float32)
+    e = engine_with(x, N)
+    e.mesh(side, r)
+    got = e.mesh_distance_field(side)
+    e.close()
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = distance_field(x, N, side, r)
+    assert np.array_equal(got, want)
+
+
 def test_distance_field_of_a_crowded_body_on_a_fine_grid(gpu_lib):
     """Thousands of particles in a block of voxels and 5,400,000 blocks: 16
     wavefronts for each of them. Sampled voxels, against the distance to the
